@@ -41,6 +41,16 @@ hipError_t launch_stage2(const uint8_t* Cq, const float* Cs, const uint8_t* w2p,
                          const int32_t* route_token, float* Y, uint16_t* out, int T, int e_local, int max_routes,
                          int32_t* queue, hipStream_t stream);
 
+// The same with 256 x 256 tiles and LDS-direct loads (prefill_wide.hip), which
+// launch_stage1 / launch_stage2 choose for large batches.
+hipError_t launch_stage1_wide(const uint8_t* hidden, const float* hs, const uint8_t* w13p, const float* w13s,
+                              const int32_t* counts, const int32_t* offsets, const int32_t* route_token, uint8_t* Cq,
+                              float* Cs, int T, int e_local, int max_routes, int32_t* queue, hipStream_t stream);
+hipError_t launch_stage2_wide(const uint8_t* Cq, const float* Cs, const uint8_t* w2p, const float* w2s,
+                              const int32_t* counts, const int32_t* offsets, const float* rw,
+                              const int32_t* route_token, float* Y, uint16_t* out, int T, int e_local, int max_routes,
+                              int32_t* queue, hipStream_t stream);
+
 // Decode path (T <= DECODE_MAX_T): GEMM1 + SwiGLU with the local dispatch
 // fused in (fp32 output Cf), the FP8 requant, then GEMM2 over 64-row items.
 hipError_t launch_stage1_decode(const int32_t* topk_ids, const float* topk_w, int T, int e_local, int offset,

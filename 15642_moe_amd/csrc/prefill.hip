@@ -1,5 +1,5 @@
-// Prefill-path grouped FP8 GEMMs (T > DECODE_MAX_T) on
-// v_mfma_f32_32x32x64_f8f6f4.
+// Prefill-path grouped FP8 GEMMs (T > DECODE_MAX_T; large batches:
+// prefill_wide.hip) on v_mfma_f32_32x32x64_f8f6f4.
 //
 // stage1_tile_kernel : G = A_e x W13_e^T with per-128-K block scales
 //     hidden_scale[kb, tok] * W13_scale[e, nb or 16+nb, kb]
@@ -367,18 +367,17 @@ stage1_tile_kernel(const uint8_t* __restrict__ hidden, const float* __restrict__
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  load_tile_table<BM>(counts, offsets, e_local, s_tp, s_cnt, s_off);
-
   const int nq = min(XCDS, (int)gridDim.x), q = blockIdx.x % nq;
+  load_tile_table<BM>(counts, offsets, e_local, s_tp, s_cnt, s_off);
   const int n_work = s_tp[e_local] * IB;
+  ItemQueue iq{nq, n_work, q, 0};
+  if (tid == 0) iq.claim(queue);
   const uint32_t alane = a_lane_offset(lane);
 
   // Thread 0 takes the next item from the queue as soon as the current
   // item's K loop is done, so the atomic's round trip runs under the
   // epilogue (taken any earlier, the claim would hold an item back from a
   // workgroup that frees up first).
-  ItemQueue iq{nq, n_work, q, 0};
-  if (tid == 0) iq.claim(queue);
   for (;;) {
     if (tid == 0) s_item = iq.next(queue);
     __syncthreads();
@@ -567,14 +566,13 @@ stage2_tile_kernel(const uint8_t* __restrict__ Cq, const float* __restrict__ Cs,
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  load_tile_table<BM>(counts, offsets, e_local, s_tp, s_cnt, s_off);
-
   const int nq = min(XCDS, (int)gridDim.x), q = blockIdx.x % nq;
+  load_tile_table<BM>(counts, offsets, e_local, s_tp, s_cnt, s_off);
   const int n_work = s_tp[e_local] * NHP;
-  const uint32_t alane = a_lane_offset(lane);
-
   ItemQueue iq{nq, n_work, q, 0};
   if (tid == 0) iq.claim(queue);
+  const uint32_t alane = a_lane_offset(lane);
+
   for (;;) {
     if (tid == 0) s_item = iq.next(queue);
     __syncthreads();
@@ -736,7 +734,8 @@ stage2_tile_kernel(const uint8_t* __restrict__ Cq, const float* __restrict__ Cs,
 
 // GEMM1 tile for a launch from the expected routes per local expert
 // (T * 8 / 256 under uniform routing; skewed routing only adds tiles):
-// 128-route tiles up to 128 expected routes, 192-route tiles above.
+// 128-route tiles up to 128 expected routes, 192-route tiles above.  (Large
+// batches over 16 or more local experts run in prefill_wide.hip.)
 bool stage1_wide_tiles(int T) { return T / 32 > 128; }
 
 // GEMM2 takes 128-route tiles up to T = 1024 and 192-route tiles above.  At
@@ -772,12 +771,25 @@ hipError_t run_stage2_tile(const uint8_t* Cq, const float* Cs, const uint8_t* w2
   return hipGetLastError();
 }
 
+// Large batches take the 256 x 256-tile kernels of prefill_wide.hip: from 96
+// expected routes per local expert (T / 32) on, and with at least 16 local
+// experts.  Measured, wide against these kernels (whole forward): even routing
+// T=2048 315 / 304 us, 2500 319 / 311, 3500 344 / 344, 4096 358 / 418, 6000 413 /
+// 494; uneven T=1500 269 / 257, 3001 331 / 338; with 16 local experts T=5000
+// 220 / 221 and T=16384 512 / 546.  With 8 local experts a 256-row item per
+// weight block leaves CUs without work unless the routing is skewed: T=4096
+// 163 / 143, T=8192 207 / 199, skewed T=4096 835 / 936.
+bool wide_path(int T, int e_local) { return T >= 3072 && e_local >= 16; }
+
 }  // namespace
 
 hipError_t launch_stage1(const uint8_t* hidden, const float* hidden_scale, const uint8_t* w13p,
                          const float* w13_scale, const int32_t* counts, const int32_t* offsets,
                          const int32_t* route_token, uint8_t* Cq, float* Cs, int T, int e_local, int max_routes,
                          int32_t* queue, hipStream_t stream) {
+  if (wide_path(T, e_local))
+    return launch_stage1_wide(hidden, hidden_scale, w13p, w13_scale, counts, offsets, route_token, Cq, Cs, T, e_local,
+                              max_routes, queue, stream);
   if (!stage1_wide_tiles(T))
     return run_stage1_tile<4, 2, 2>(hidden, hidden_scale, w13p, w13_scale, counts, offsets, route_token, Cq, Cs, T,
                                     e_local, max_routes, queue, stream);
@@ -790,6 +802,9 @@ hipError_t launch_stage2(const uint8_t* Cq, const float* Cs, const uint8_t* w2p,
                          const int32_t* route_token, float* Y, uint16_t* out,
                          int T, int e_local, int max_routes, int32_t* queue,
                          hipStream_t stream) {
+  if (wide_path(T, e_local))
+    return launch_stage2_wide(Cq, Cs, w2p, w2_scale, counts, offsets, route_weight, route_token, Y, out, T, e_local,
+                              max_routes, queue, stream);
   if (stage2_narrow_tiles(T))
     return run_stage2_tile<4, 2, 1>(Cq, Cs, w2p, w2_scale, counts, offsets, route_weight, route_token, Y, out, e_local,
                                     max_routes, queue, stream);

@@ -466,6 +466,36 @@ def test_forward_skewed_either_side_of_the_gemm2_tile_switch(ops, cuda, T):
     _check_against_models(f"skewed T={T}", out, _cpu(inp))
 
 
+@pytest.mark.parametrize("T,e_local,hot", [(3071, 32, 0), (3072, 32, 0), (3072, 16, 0), (3333, 17, 3), (3100, 31, 9)])
+def test_forward_wide_prefill_tiles(ops, cuda, T, e_local, hot):
+    """The wide prefill GEMMs (T >= 3072 and 16 or more local experts) and
+    the last T below them.  hot > 0: exact route counts at the edges of
+    fragments, tiles and bands on the first experts (each token's other
+    picks are spread over the rest), so that some experts have 0, 1, 32, 33,
+    256, 257 and more than eight tiles' worth of routes."""
+    from conftest import pkg
+
+    layer = pkg("moe_layer")
+    inp = layer.build_moe_inputs(T=T, device="cuda", seed=T + e_local)
+    for k in ("gemm1_weights", "gemm1_weights_scale", "gemm2_weights", "gemm2_weights_scale"):
+        inp[k] = inp[k][:e_local].contiguous()
+    if hot:
+        edges = [1, 32, 33, 0, 256, 257, 31, 289, T][:hot] if hot > 3 else [T, 2049, 33]
+        logits = torch.randn(T, 256, generator=torch.Generator().manual_seed(T)) - 12.0
+        logits[:, 224:] += 20.0  # every token's remaining picks, outside the local experts
+        for e, n in enumerate(edges):
+            logits[:n, e] += 40.0
+        for e in range(len(edges), e_local):
+            logits[:, e] -= 40.0
+        inp["routing_logits"] = logits.to("cuda")
+    print(f"[forward] wide prefill T={T} E_local={e_local} hot={hot}", flush=True)
+    out = layer.run_custom(ops, **inp)
+    out2 = layer.run_custom(ops, **inp)
+    torch.cuda.synchronize()
+    _check_against_models(f"wide prefill T={T} E={e_local}", out, _cpu(inp))
+    assert torch.equal(out.view(torch.int16), out2.view(torch.int16))
+
+
 @pytest.mark.parametrize("case", range(6))
 def test_forward_random_shapes(ops, cuda, case):
     """Seeded random (T, local_expert_offset, E_local, routed_scaling_factor)

@@ -222,3 +222,50 @@ def test_item_queue_protocol_claims_every_item_once(seed):
             assert claims <= items_of[p] + nq + 1
             del live[p]
     assert sorted(taken) == list(range(n_work))
+
+
+def _wide_order(counts, frags, U):
+    """Queue lists of prefill_wide.hip's WideWork for one tile size."""
+    f = [(c + 31) // 32 for c in counts] + [0] * (32 - len(counts))
+    nt = [-(-x // frags) for x in f]
+    key = [-(-x // n) if n else 0 for x, n in zip(f, nt)]
+    order = sorted(range(32), key=lambda e: (-key[e], e))
+    queues = []
+    for x in range(8):
+        items = []
+        for i in range(32):
+            p = 31 - i if x & 1 else i
+            if (x - U * p) % 8 >= U:
+                continue
+            e, n = order[p], nt[order[p]]
+            full = n // 8
+            for local in range(4 * n):
+                band = local // 32
+                width = 8 if band < full else n - full * 8
+                r = local - min(band, full) * 32
+                mt = min(band, full) * 8 + r % width
+                items.append((e, 4 * ((x - U * p) % 8) + r // width, mt))
+        queues.append(items)
+    return queues, f, nt
+
+
+@pytest.mark.parametrize("seed", range(24))
+def test_wide_work_lists_every_item_once(seed):
+    """The wide prefill GEMMs' work lists: for any route counts and tile size,
+    every (expert, weight block, route tile) is in exactly one queue, and an
+    expert's route tiles partition its routes, none of more than the tile size."""
+    rng = np.random.default_rng(seed)
+    n = int(rng.integers(1, 33))
+    counts = [int(c) for c in rng.choice([0, 1, 31, 32, 33, 255, 256, 257, 513, 2304, 2305, 4096], size=n)]
+    frags = int(rng.choice([8, 6, 4, 3, 2]))
+    for U in (4, 7):
+        queues, f, nt = _wide_order(counts, frags, U)
+        got = sorted(it for q in queues for it in q)
+        assert got == sorted((e, b, m) for e in range(32) for b in range(4 * U) for m in range(nt[e]))
+    for e, c in enumerate(counts):
+        at = 0
+        for m in range(nt[e]):
+            lo, hi = 32 * (m * f[e] // nt[e]), min(c, 32 * ((m + 1) * f[e] // nt[e]))
+            assert lo == at and 0 < hi - lo <= 32 * frags
+            at = hi
+        assert at == c

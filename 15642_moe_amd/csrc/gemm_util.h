@@ -68,21 +68,29 @@ __device__ __forceinline__ v8i load_tile_frag(const uint8_t* __restrict__ tile, 
 }
 
 // Per-workgroup table of route tiles per local expert: expert e owns route
-// tiles s_tp[e] .. s_tp[e+1]-1 of BM routes each.
+// tiles s_tp[e] .. s_tp[e+1]-1 of BM routes each.  Lane e of the first wave
+// reads expert e's count and offset and a 32-lane scan sums the tiles: one
+// memory latency, where one thread walking the experts took 32 dependent
+// LDS writes after it at the start of every launch.
 template <int BM>
 __device__ __forceinline__ void load_tile_table(const int32_t* __restrict__ counts,
                                                 const int32_t* __restrict__ offsets, int e_local, int* s_tp,
                                                 int* s_cnt, int* s_off) {
-  if (threadIdx.x == 0) {
-    int acc = 0;
-    for (int e = 0; e < e_local; ++e) {
-      const int c = counts[e];
-      s_cnt[e] = c;
-      s_off[e] = offsets[e];
-      s_tp[e] = acc;
-      acc += (c + BM - 1) / BM;
+  if (threadIdx.x < MAX_E_LOCAL) {
+    const int e = threadIdx.x;
+    const int c = e < e_local ? counts[e] : 0, o = e < e_local ? offsets[e] : 0;
+    int inc = (c + BM - 1) / BM;
+#pragma unroll
+    for (int d = 1; d < MAX_E_LOCAL; d <<= 1) {
+      const int x = __shfl_up(inc, d, MAX_E_LOCAL);
+      if (e >= d) inc += x;
     }
-    s_tp[e_local] = acc;
+    if (e < e_local) {
+      s_cnt[e] = c;
+      s_off[e] = o;
+      s_tp[e + 1] = inc;
+    }
+    if (e == 0) s_tp[0] = 0;
   }
   __syncthreads();
 }

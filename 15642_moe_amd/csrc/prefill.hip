@@ -368,10 +368,12 @@ stage1_tile_kernel(const uint8_t* __restrict__ hidden, const float* __restrict__
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int nq = min(XCDS, (int)gridDim.x), q = blockIdx.x % nq;
+  // The first claim's round trip runs under the table's loads.
+  ItemQueue iq{nq, 0, q, 0};
+  if (tid == 0) iq.claim(queue);
   load_tile_table<BM>(counts, offsets, e_local, s_tp, s_cnt, s_off);
   const int n_work = s_tp[e_local] * IB;
-  ItemQueue iq{nq, n_work, q, 0};
-  if (tid == 0) iq.claim(queue);
+  iq.n_work = n_work;
   const uint32_t alane = a_lane_offset(lane);
 
   // Thread 0 takes the next item from the queue as soon as the current
@@ -567,10 +569,11 @@ stage2_tile_kernel(const uint8_t* __restrict__ Cq, const float* __restrict__ Cs,
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int nq = min(XCDS, (int)gridDim.x), q = blockIdx.x % nq;
+  ItemQueue iq{nq, 0, q, 0};  // first claim as in stage 1
+  if (tid == 0) iq.claim(queue);
   load_tile_table<BM>(counts, offsets, e_local, s_tp, s_cnt, s_off);
   const int n_work = s_tp[e_local] * NHP;
-  ItemQueue iq{nq, n_work, q, 0};
-  if (tid == 0) iq.claim(queue);
+  iq.n_work = n_work;
   const uint32_t alane = a_lane_offset(lane);
 
   for (;;) {

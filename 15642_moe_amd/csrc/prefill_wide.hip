@@ -50,18 +50,21 @@ struct WideGeom {
 // LDS address lds + 16 l (4 l).  M0 holds the LDS address; the kernels use it
 // for nothing else.  They are counted by vmcnt like any load, and the
 // compiler knows nothing of them: every wait is explicit (landed_barrier,
-// wait_loads).  NTL: non-temporal.
+// wait_loads).  The wait states in front also cover a base address that a
+// VALU instruction has just written (the reload of a spilled scalar register;
+// five states to its use by a memory instruction, which the compiler does not
+// insert for inline assembly).  NTL: non-temporal.
 template <bool NTL>
 __device__ __forceinline__ void dma16(uint32_t lds, uint32_t voff, const void* sbase) {
   if constexpr (NTL)
-    __asm__ volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt" ::"s"(lds), "v"(voff), "s"(sbase)
+    __asm__ volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tglobal_load_lds_dwordx4 %1, %2 nt" ::"s"(lds), "v"(voff), "s"(sbase)
                      : "memory");
   else
-    __asm__ volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(voff), "s"(sbase)
+    __asm__ volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(voff), "s"(sbase)
                      : "memory");
 }
 __device__ __forceinline__ void dma4(uint32_t lds, uint32_t voff, const void* sbase) {
-  __asm__ volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(lds), "v"(voff), "s"(sbase)
+  __asm__ volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tglobal_load_lds_dword %1, %2" ::"s"(lds), "v"(voff), "s"(sbase)
                    : "memory");
 }
 // All but this wave's N youngest loads have landed and its LDS reads are done;

@@ -19,19 +19,30 @@
 #include "gemm_util.h"
 #include "launch.h"
 
+#include <type_traits>
+
 namespace moe {
 
 // ---------------------------------------------------------------------------
 // Decode variants (small T).  Streaming the weights of the hit experts is the
 // whole cost, and a CU streams at a bounded rate (~35-40 GB/s), so the work is
-// cut into thousands of single-wave items (one per (expert, weight slice))
-// that spread evenly over the 256 CUs.  Each wave loads its weight tiles and
-// the 16-route activation fragment straight into registers through an
-// NR-deep ring: no LDS and no barrier in the K loop.  A static grid covers
-// every (expert, slice) pair in expert-major order; since workgroup p runs on
-// XCD p % 8, every expert's slices are dealt round-robin over all XCDs, so the
-// load stays even whichever experts the routing hits.  Experts without routes
-// exit at once.
+// cut into thousands of items (one per (expert, weight slice)) that spread
+// evenly over the 256 CUs.  Each wave loads its weight tiles and the 16-route
+// activation fragment straight into registers through an NR-deep ring: no LDS
+// and no barrier in the K loop.  Where items are few or short, KW waves of a
+// workgroup take a part of the item's K-blocks each and the first adds the
+// parts in K order: more loads in flight per item, and a part that fits the
+// ring has all of them in flight at once.  GEMM2's 16 K-blocks by four waves,
+// whole call: T=64 uneven 136 -> 135 us, T=96 224 -> 215, T=113 even 225 ->
+// 217, skewed T=128 323 -> 308.
+// Items are dealt expert-major over the experts that have routes, found from
+// the picks (GEMM1) or counts (GEMM2) by every workgroup; since workgroup p
+// runs on XCD p % 8, every expert's slices are dealt round-robin over all
+// XCDs.  The grid holds the experts that T tokens can hit at most, and
+// workgroups past the hit ones exit at once.  (With a static grid over all
+// experts and a 32-step count loop in each workgroup the empty ones cost as
+// much as the streaming at small T: T=4 54 -> 41 us, T=8 73 -> 60, T=16
+// 70 -> 55, T=32 90 -> 80 without them.)
 // ---------------------------------------------------------------------------
 
 // Lane k's value of v (k wave-uniform): the weight-block scales sit one
@@ -40,22 +51,51 @@ __device__ __forceinline__ float lane_value(float v, int k) {
   return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), k));
 }
 
-__device__ __forceinline__ void decode_map(int p, int nslice, int& e, int& slice) {
-  e = p / nslice;
-  slice = p - e * nslice;
+// OR / sum over the wave's lanes, a uniform value: within rows of 16 lanes by
+// DPP (lanes l ^ 1, l ^ 2, l ^ 7, l ^ 15), over the rows by readlane.
+template <class Op>
+__device__ __forceinline__ uint32_t wave_reduce_u32(uint32_t x, Op op) {
+  x = op(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0xB1, 0xF, 0xF, false));
+  x = op(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x4E, 0xF, 0xF, false));
+  x = op(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x141, 0xF, 0xF, false));
+  x = op(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x140, 0xF, 0xF, false));
+  const uint32_t r0 = (uint32_t)__builtin_amdgcn_readlane((int)x, 0), r1 = (uint32_t)__builtin_amdgcn_readlane((int)x, 16);
+  const uint32_t r2 = (uint32_t)__builtin_amdgcn_readlane((int)x, 32), r3 = (uint32_t)__builtin_amdgcn_readlane((int)x, 48);
+  return op(op(r0, r1), op(r2, r3));
 }
 
-// Stage 1, one wave per (expert e, NPW gate/up tile pairs from j*NPW): 16*NPW
+// Item p -> (expert, slice): the experts that `hits` marks in ascending
+// order, nslice items each.  False past the last one.
+__device__ __forceinline__ bool decode_map(int p, int nslice, uint32_t hits, int& e, int& slice) {
+  const int i = p / nslice;
+  if (i >= __popc(hits)) return false;
+  for (int k = 0; k < i; ++k) hits &= hits - 1;
+  e = __builtin_ctz(hits);
+  slice = p - i * nslice;
+  return true;
+}
+
+// f(integral_constant<int, 0>{}) .. f(integral_constant<int, N - 1>{}).
+template <int N, int I0 = 0, class F>
+__device__ __forceinline__ void static_for(F&& f) {
+  if constexpr (I0 < N) {
+    f(std::integral_constant<int, I0>{});
+    static_for<N, I0 + 1>(f);
+  }
+}
+
+// Stage 1, KW waves per (expert e, NPW gate/up tile pairs from j*NPW): 16*NPW
 // I columns (each activation fragment serves 2*NPW weight tiles),
 // c = gate * silu(up) written in fp32 to Cf [R, 2048] (the FP8 requant needs
 // the amax over 128 columns, i.e. over several items, and runs in
 // quant_kernel).  The
-// local dispatch is fused into the prologue: every item ranks the T x 8 picks
-// with wave ballots (counts, offsets, its expert's tokens in token order);
-// items j == 0 publish their expert's route arrays, item (0, 0) the counts,
-// offsets and the -1 tails of token_route.
-template <int NR, int FR, int NPW>
-__global__ void __launch_bounds__(64)
+// local dispatch is fused into the prologue: every item takes its expert's
+// count, first route and tokens (in token order) from the T x 8 picks by wave
+// ballots and sums; items j == 0 publish their expert's route arrays, and the
+// first workgroup, which has no item, the counts, offsets and the -1 tails of
+// token_route.
+template <int NR, int FR, int NPW, int KW>
+__global__ void __launch_bounds__(64 * KW)
 stage1_decode_kernel(const int32_t* __restrict__ topk_ids, const float* __restrict__ topk_w, int T, int e_local,
                      int offset, const uint8_t* __restrict__ hidden, const float* __restrict__ hscale,
                      const uint8_t* __restrict__ w13p, const float* __restrict__ w13s, int32_t* __restrict__ counts,
@@ -63,13 +103,11 @@ stage1_decode_kernel(const int32_t* __restrict__ topk_ids, const float* __restri
                      float* __restrict__ route_weight, int32_t* __restrict__ token_route, float* __restrict__ Cf) {
   constexpr int BM = 16, NPAIR = I / 16 / NPW;
   static_assert(8 % NPW == 0, "an item's tile pairs lie in one 128-column block");
-  static_assert(HB % NR == 0, "ring depth must divide the K-block count");
+  constexpr int KPB = HB / KW;  // K-blocks per wave
+  static_assert(HB % KW == 0 && KPB % NR == 0, "the waves split the K-blocks evenly, into whole rings");
   __shared__ int s_tok[DECODE_MAX_T];
-  const int lane = threadIdx.x;
-  int e, j;
-  decode_map(blockIdx.x, NPAIR, e, j);
-  if (e >= e_local) return;
-
+  __shared__ v4f s_part[KW > 1 ? KW - 1 : 1][FR * NPW * 2][64];
+  const int lane = threadIdx.x & 63, wave = KW > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
   // ---- dispatch: masks of the tokens this lane reads (T <= 128 -> 2 per lane)
   constexpr int TPL = DECODE_MAX_T / 64;
   uint32_t mask[TPL];
@@ -78,17 +116,16 @@ stage1_decode_kernel(const int32_t* __restrict__ topk_ids, const float* __restri
     const int t = c * 64 + lane;
     mask[c] = t < T ? local_mask(topk_ids + (size_t)t * TOP_K, offset, e_local) : 0u;
   }
-  int my_cnt = 0, my_off = 0, total = 0;
-  for (int e2 = 0; e2 < e_local; ++e2) {
-    int n = 0;
+  if (blockIdx.x == 0) {  // the first workgroup publishes counts, offsets and the -1 tails
+    if (wave > 0) return;
+    int total = 0;
+    for (int e2 = 0; e2 < e_local; ++e2) {
+      int n = 0;
 #pragma unroll
-    for (int c = 0; c < TPL; ++c) n += __popcll(__ballot((mask[c] >> e2) & 1u));
-    if (e2 < e) my_off += n;
-    if (e2 == e) my_cnt = n;
-    if (blockIdx.x == 0 && lane == 0) { counts[e2] = n; offsets[e2] = total; }
-    total += n;
-  }
-  if (blockIdx.x == 0) {
+      for (int c = 0; c < TPL; ++c) n += __popcll(__ballot((mask[c] >> e2) & 1u));
+      if (lane == 0) { counts[e2] = n; offsets[e2] = total; }
+      total += n;
+    }
     if (lane == 0) offsets[e_local] = total;
 #pragma unroll
     for (int c = 0; c < TPL; ++c) {
@@ -96,8 +133,23 @@ stage1_decode_kernel(const int32_t* __restrict__ topk_ids, const float* __restri
       if (t < T)
         for (int k = __popc(mask[c]); k < TOP_K; ++k) token_route[(size_t)t * TOP_K + k] = -1;
     }
+    return;
   }
-  if (my_cnt == 0) return;
+  uint32_t any = 0;
+#pragma unroll
+  for (int c = 0; c < TPL; ++c) any |= mask[c];
+  int e, j;
+  if (!decode_map(blockIdx.x - 1, NPAIR, wave_reduce_u32(any, [](uint32_t a, uint32_t b) { return a | b; }), e, j))
+    return;
+  // Routes of the experts below e, and of e.
+  uint32_t lower = 0;
+  int my_cnt = 0;
+#pragma unroll
+  for (int c = 0; c < TPL; ++c) {
+    lower += __popc(mask[c] & ((1u << e) - 1u));
+    my_cnt += __popcll(__ballot((mask[c] >> e) & 1u));
+  }
+  const int my_off = (int)wave_reduce_u32(lower, [](uint32_t a, uint32_t b) { return a + b; });
   const uint64_t below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
   int base = 0;
 #pragma unroll
@@ -105,7 +157,7 @@ stage1_decode_kernel(const int32_t* __restrict__ topk_ids, const float* __restri
     const int t = c * 64 + lane;
     const bool hit = (mask[c] >> e) & 1u;
     const uint64_t bal = __ballot(hit);
-    if (hit) {
+    if (hit && wave == 0) {
       const int slot = base + __popcll(bal & below);
       s_tok[slot] = t;
       if (j == 0) {
@@ -127,6 +179,7 @@ stage1_decode_kernel(const int32_t* __restrict__ topk_ids, const float* __restri
   const v4f zero4 = {0.f, 0.f, 0.f, 0.f};
   const int col = lane & 15;
   const int nb = (j * NPW) >> 3, pj = (j * NPW) & 7;
+  const int k0 = wave * KPB, k1 = k0 + KPB;  // this wave's K-blocks
   const uint8_t* wp = w13p + (size_t)(e * IB + nb) * W13_SLAB_BYTES + (size_t)(2 * pj) * TILE_BYTES;
   const float* wsg_p = w13s + (size_t)(e * G1B + nb) * HB;
   const float* wsu_p = w13s + (size_t)(e * G1B + IB + nb) * HB;
@@ -171,20 +224,24 @@ stage1_decode_kernel(const int32_t* __restrict__ topk_ids, const float* __restri
       }
     };
     wait_vm<0>();  // the ring starts from an empty vmcnt queue: its waits count only its own loads
+    // A part that fits the ring is all issued here; a longer one keeps NR
+    // K-blocks in flight.
+    constexpr bool ONE = KPB == NR;
 #pragma unroll
-    for (int sl = 0; sl < NR - 1; ++sl) issue(sl, sl);
+    for (int sl = 0; sl < (ONE ? NR : NR - 1); ++sl) issue(k0 + sl, sl);
     v4f accg[FR][NPW], accu[FR][NPW];
 #pragma unroll
     for (int f = 0; f < FR; ++f)
 #pragma unroll
       for (int p = 0; p < NPW; ++p) { accg[f][p] = zero4; accu[f][p] = zero4; }
 #pragma unroll 1
-    for (int kb0 = 0; kb0 < HB; kb0 += NR) {
-#pragma unroll
-      for (int sl = 0; sl < NR; ++sl) {
+    for (int kb0 = k0; kb0 < k1; kb0 += NR) {
+      static_for<NR>([&](auto slc) __attribute__((always_inline)) {
+        constexpr int sl = decltype(slc)::value;
         const int kb = kb0 + sl;
-        issue(min(kb + NR - 1, HB - 1), (sl + NR - 1) % NR);  // branch-free; the tail re-reads a K-block
-        wait_vm<LPK * (NR - 1)>();
+        // branch-free; the tail re-reads a K-block
+        if constexpr (!ONE) issue(min(kb + NR - 1, k1 - 1), (sl + NR - 1) % NR);
+        wait_vm<LPK * (ONE ? NR - 1 - sl : NR - 1)>();
 #pragma unroll
         for (int p = 0; p < NPW; ++p) __asm__ volatile("" : "+v"(wgl[sl][p]), "+v"(wgh[sl][p]), "+v"(wul[sl][p]), "+v"(wuh[sl][p]));
 #pragma unroll
@@ -200,9 +257,33 @@ stage1_decode_kernel(const int32_t* __restrict__ topk_ids, const float* __restri
           }
         }
         __builtin_amdgcn_sched_barrier(0);
-      }
+      });
     }
     wait_vm_all();  // the dead tail loads land before the registers are reused
+    if constexpr (KW > 1) {
+      // The parts' sums, added in K order by the first wave.
+      if (m0 > 0) __syncthreads();  // it has read the previous pass's
+      if (wave > 0) {
+#pragma unroll
+        for (int f = 0; f < FR; ++f)
+#pragma unroll
+          for (int p = 0; p < NPW; ++p) {
+            s_part[wave - 1][(f * NPW + p) * 2][lane] = accg[f][p];
+            s_part[wave - 1][(f * NPW + p) * 2 + 1][lane] = accu[f][p];
+          }
+      }
+      __syncthreads();
+      if (wave > 0) continue;
+#pragma unroll
+      for (int k = 0; k < KW - 1; ++k)
+#pragma unroll
+        for (int f = 0; f < FR; ++f)
+#pragma unroll
+          for (int p = 0; p < NPW; ++p) {
+            accg[f][p] += s_part[k][(f * NPW + p) * 2][lane];
+            accu[f][p] += s_part[k][(f * NPW + p) * 2 + 1][lane];
+          }
+    }
 #pragma unroll
     for (int f = 0; f < FR; ++f) {
       if (col < rows[f]) {
@@ -247,24 +328,27 @@ quant_kernel(const float* __restrict__ Cf, const int32_t* __restrict__ offsets, 
   }
 }
 
-// Stage 2, one wave per (expert e, 64-row H slice q): tiles 4*(q%2)..+3 of
+// Stage 2, KW waves per (expert e, 64-row H slice q): tiles 4*(q%2)..+3 of
 // the 128-row slab hb = q/2.
-template <int NR, int FR>
-__global__ void __launch_bounds__(64)
+template <int NR, int FR, int KW>
+__global__ void __launch_bounds__(64 * KW)
 stage2_decode_kernel(const uint8_t* __restrict__ Cq, const float* __restrict__ Cs, const uint8_t* __restrict__ w2p,
                      const float* __restrict__ w2s, const int32_t* __restrict__ counts,
                      const int32_t* __restrict__ offsets, const float* __restrict__ route_weight,
                      const int32_t* __restrict__ route_token, float* __restrict__ Y, uint16_t* __restrict__ out,
                      int e_local) {
   constexpr int BM = 16, NSLICE = H / 64;
-  static_assert(IB % NR == 0, "ring depth must divide the K-block count");
-  const int lane = threadIdx.x;
+  constexpr int KPB = IB / KW;  // K-blocks per wave
+  static_assert(IB % KW == 0 && KPB % NR == 0, "the waves split the K-blocks evenly, into whole rings");
+  __shared__ v4f s_part[KW > 1 ? KW - 1 : 1][FR * 4][64];
+  const int lane = threadIdx.x & 63, wave = KW > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
+  const int k0 = wave * KPB, k1 = k0 + KPB;  // this wave's K-blocks
+  // Lane l reads expert l's count and offset: one latency for both.
+  const int el = lane < e_local ? lane : 0;
+  const int cnt_l = counts[el], off_l = offsets[el];
   int e, q;
-  decode_map(blockIdx.x, NSLICE, e, q);
-  if (e >= e_local) return;
-  const int cnt = counts[e];
-  if (cnt == 0) return;
-  const int off = offsets[e];
+  if (!decode_map(blockIdx.x, NSLICE, (uint32_t)__ballot(lane < e_local && cnt_l > 0), e, q)) return;
+  const int cnt = __builtin_amdgcn_readlane(cnt_l, e), off = __builtin_amdgcn_readlane(off_l, e);
   const int hb = q >> 1, t0 = 4 * (q & 1);
   const uint8_t* wp = w2p + (size_t)(e * HB + hb) * W2_SLAB_BYTES + (size_t)t0 * TILE_BYTES;
   const float* ws_p = w2s + (size_t)(e * HB + hb) * IB;
@@ -304,20 +388,21 @@ stage2_decode_kernel(const uint8_t* __restrict__ Cq, const float* __restrict__ C
       }
     };
     wait_vm<0>();  // the ring starts from an empty vmcnt queue: its waits count only its own loads
+    constexpr bool ONE = KPB == NR;  // as in stage 1
 #pragma unroll
-    for (int sl = 0; sl < NR - 1; ++sl) issue(sl, sl);
+    for (int sl = 0; sl < (ONE ? NR : NR - 1); ++sl) issue(k0 + sl, sl);
     v4f acc[FR][4];
 #pragma unroll
     for (int f = 0; f < FR; ++f)
 #pragma unroll
       for (int i = 0; i < 4; ++i) acc[f][i] = zero4;
 #pragma unroll 1
-    for (int kb0 = 0; kb0 < IB; kb0 += NR) {
-#pragma unroll
-      for (int sl = 0; sl < NR; ++sl) {
+    for (int kb0 = k0; kb0 < k1; kb0 += NR) {
+      static_for<NR>([&](auto slc) __attribute__((always_inline)) {
+        constexpr int sl = decltype(slc)::value;
         const int kb = kb0 + sl;
-        issue(min(kb + NR - 1, IB - 1), (sl + NR - 1) % NR);  // branch-free, clamped
-        wait_vm<LPK * (NR - 1)>();
+        if constexpr (!ONE) issue(min(kb + NR - 1, k1 - 1), (sl + NR - 1) % NR);  // branch-free, clamped
+        wait_vm<LPK * (ONE ? NR - 1 - sl : NR - 1)>();
         __asm__ volatile("" : "+v"(wl[sl][0]), "+v"(wh[sl][0]), "+v"(wl[sl][1]), "+v"(wh[sl][1]), "+v"(wl[sl][2]),
                          "+v"(wh[sl][2]), "+v"(wl[sl][3]), "+v"(wh[sl][3]));
 #pragma unroll
@@ -333,9 +418,26 @@ stage2_decode_kernel(const uint8_t* __restrict__ Cq, const float* __restrict__ C
           }
         }
         __builtin_amdgcn_sched_barrier(0);
-      }
+      });
     }
     wait_vm_all();
+    if constexpr (KW > 1) {  // as in stage 1
+      if (m0 > 0) __syncthreads();
+      if (wave > 0) {
+#pragma unroll
+        for (int f = 0; f < FR; ++f)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) s_part[wave - 1][f * 4 + i][lane] = acc[f][i];
+      }
+      __syncthreads();
+      if (wave > 0) continue;
+#pragma unroll
+      for (int k = 0; k < KW - 1; ++k)
+#pragma unroll
+        for (int f = 0; f < FR; ++f)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) acc[f][i] += s_part[k][f * 4 + i][lane];
+    }
 #pragma unroll
     for (int f = 0; f < FR; ++f) {
       if (col < rows[f]) {
@@ -430,26 +532,34 @@ hipError_t launch_mfma_ceiling(float* out, unsigned long long* clocks, int iters
 // ---------------------------------------------------------------------------
 // Host launchers.
 // ---------------------------------------------------------------------------
+// The most local experts that T tokens can hit.
+static int decode_experts(int T, int e_local) { return T * TOP_K < e_local ? T * TOP_K : e_local; }
+
 hipError_t launch_stage1_decode(const int32_t* topk_ids, const float* topk_w, int T, int e_local, int offset,
                                 const uint8_t* hidden, const float* hidden_scale, const uint8_t* w13p,
                                 const float* w13_scale, int32_t* counts, int32_t* offsets, int32_t* route_token,
                                 float* route_weight, int32_t* token_route, float* Cf, uint8_t* Cq, float* Cs,
                                 hipStream_t stream) {
   if (T > DECODE_MAX_T) return hipErrorInvalidValue;
-  constexpr int NPW = 2;
-  const int grid = e_local * (I / 16 / NPW);
-  // Two fragments per weight pass once experts can hold more than 16
-  // routes often enough to matter; at T <= 64 one (its registers keep two
-  // waves per SIMD either way, but the second fragment's loads would be
-  // padding for nearly every item).
+  auto launch = [&](auto kernel, int npw, int kw) {
+    kernel<<<1 + decode_experts(T, e_local) * (I / 16 / npw), 64 * kw, 0, stream>>>(
+        topk_ids, topk_w, T, e_local, offset, hidden, hidden_scale, w13p, w13_scale, counts, offsets, route_token,
+        route_weight, token_route, Cf);
+  };
+  // Up to 32 tokens one tile pair per wave: the items are few and their
+  // number, not the prologue, sets the balance (whole call, two pairs ->
+  // one: T=4 40.5 -> 39.7 us, T=16 56.9 -> 55.4, T=32 79.8 -> 77.5).  Up to
+  // 64 two waves share such an item's K range (T=48 one wave 135.6, two
+  // 133.6; T=64 even 185.0 and 181.0, uneven 133.0 and 130.8).  Above, hot
+  // experts hold several fragments: two per weight pass and two pairs per
+  // wave (skewed T=90 263 us, where one fragment and one pair take 321;
+  // even T=113 218 and 213).
   if (T > 64)
-    stage1_decode_kernel<4, 2, NPW><<<grid, 64, 0, stream>>>(topk_ids, topk_w, T, e_local, offset, hidden, hidden_scale,
-                                                        w13p, w13_scale, counts, offsets, route_token, route_weight,
-                                                        token_route, Cf);
+    launch(stage1_decode_kernel<4, 2, 2, 1>, 2, 1);
+  else if (T > 32)
+    launch(stage1_decode_kernel<4, 1, 1, 2>, 1, 2);
   else
-    stage1_decode_kernel<4, 1, NPW><<<grid, 64, 0, stream>>>(topk_ids, topk_w, T, e_local, offset, hidden, hidden_scale,
-                                                        w13p, w13_scale, counts, offsets, route_token, route_weight,
-                                                        token_route, Cf);
+    launch(stage1_decode_kernel<4, 1, 1, 1>, 1, 1);
   hipError_t err = hipGetLastError();
   if (err != hipSuccess) return err;
   const int R = T * (e_local < TOP_K ? e_local : TOP_K);
@@ -461,13 +571,16 @@ hipError_t launch_stage2_decode(const uint8_t* Cq, const float* Cs, const uint8_
                                 const int32_t* counts, const int32_t* offsets, const float* route_weight,
                                 const int32_t* route_token, float* Y, uint16_t* out, int e_local, int T,
                                 hipStream_t stream) {
-  const int grid = e_local * (H / 64);
-  if (T > 64)  // as stage 1: two fragments per weight pass
-    stage2_decode_kernel<4, 2><<<grid, 64, 0, stream>>>(Cq, Cs, w2p, w2_scale, counts, offsets, route_weight,
-                                                        route_token, Y, out, e_local);
+  const int grid = decode_experts(T, e_local) * (H / 64);
+  // An expert holds at most T routes: one fragment up to 16 tokens, two per
+  // weight pass above (skewed T=30 106 -> 99 us for the whole call, skewed
+  // T=64 261 -> 245; even T=32 79.8 -> 81.2).
+  if (T > 16)
+    stage2_decode_kernel<4, 2, 4><<<grid, 256, 0, stream>>>(Cq, Cs, w2p, w2_scale, counts, offsets, route_weight,
+                                                            route_token, Y, out, e_local);
   else
-    stage2_decode_kernel<4, 1><<<grid, 64, 0, stream>>>(Cq, Cs, w2p, w2_scale, counts, offsets, route_weight,
-                                                        route_token, Y, out, e_local);
+    stage2_decode_kernel<4, 1, 4><<<grid, 256, 0, stream>>>(Cq, Cs, w2p, w2_scale, counts, offsets, route_weight,
+                                                            route_token, Y, out, e_local);
   return hipGetLastError();
 }
 

@@ -447,6 +447,34 @@ def test_forward_every_token_on_the_same_experts(ops, cuda, T):
     _check_against_models(f"same experts T={T}", out, _cpu(inp))
 
 
+@pytest.mark.parametrize("T,e_local,experts", [
+    (1, 32, [31]), (1, 1, [0]), (2, 32, [0, 31]), (3, 9, [2, 8]), (16, 32, [5]), (17, 32, [5, 6, 30]),
+    (32, 32, [0, 1, 17, 31]), (33, 32, [0, 17]), (64, 13, [12]), (65, 32, [3, 31]), (128, 3, [1])])
+def test_forward_decode_items(ops, cuda, T, e_local, experts):
+    """The decode kernels either side of each switch by T, with routes on few
+    and distant local experts (items are dealt over the hit ones): every
+    token picks `experts` (the first one only by all but the last token) and
+    experts outside the rank."""
+    from conftest import pkg
+
+    layer = pkg("moe_layer")
+    inp = layer.build_moe_inputs(T=T, device="cuda", seed=T + e_local)
+    for k in ("gemm1_weights", "gemm1_weights_scale", "gemm2_weights", "gemm2_weights_scale"):
+        inp[k] = inp[k][:e_local].contiguous()
+    logits = torch.randn(T, 256, generator=torch.Generator().manual_seed(T)) - 12.0
+    logits[:, 224:] += 20.0  # every token's remaining picks, outside the local experts
+    logits[:, experts] = 30.0 + torch.rand(T, len(experts), generator=torch.Generator().manual_seed(T + 1))
+    if T > 1 and len(experts) > 1:
+        logits[-1, experts[0]] = -40.0
+    inp["routing_logits"] = logits.to("cuda")
+    print(f"[forward] decode items T={T} E_local={e_local} experts={experts}", flush=True)
+    out = layer.run_custom(ops, **inp)
+    out2 = layer.run_custom(ops, **inp)
+    torch.cuda.synchronize()
+    _check_against_models(f"decode items T={T} E={e_local}", out, _cpu(inp))
+    assert torch.equal(out.view(torch.int16), out2.view(torch.int16))
+
+
 @pytest.mark.parametrize("T", [1024, 1025])
 def test_forward_skewed_either_side_of_the_gemm2_tile_switch(ops, cuda, T):
     """Routing bias +3 on local experts 0-3 (as config 4) at T = 1024 (GEMM2

@@ -11,13 +11,14 @@
 // builder (moe_layer.py:45-75).  The quantisation rule is the path's own
 // requant rule (kernels/moe.cu:516-541).
 //
-// One workgroup covers 64 tokens x 64 experts (a quarter of the router) x a
-// range of K-blocks.  Per 128-column K-block its 256 threads gather the 64
+// One workgroup covers 64 tokens x 64, 128 or 256 experts (one 16-expert tile
+// per wave: 4, 8 or 16 waves) x a range of K-blocks.  Per 128-column K-block
+// its threads gather the 64
 // token rows (16 lanes per row: two whole cache lines), the block is staged
 // in LDS in the B-operand layout of v_mfma_f32_16x16x32_bf16, and each wave
 // multiplies it with its 16-expert tile of the packed router weight (A
-// operand, streamed from L2: the whole weight is 3.5 MiB).  Each of the four
-// expert-quarter workgroups of a token tile also quantises 16 of its rows
+// operand, streamed from L2: the whole weight is 3.5 MiB).  The
+// workgroups of a token tile (expert parts) each quantise their share of its rows
 // (the 16 lanes of a row hold the whole 128-column block, so the amax is a
 // 16-lane shuffle reduction).  Loads run three K-blocks ahead through a
 // 4-slot register ring.  Small T splits K over workgroups; their partial
@@ -34,8 +35,8 @@ namespace {
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 
 constexpr int RQ_TOK = 64;                       // tokens per workgroup (4 tiles of 16)
-constexpr int RQ_EQ = 4;                         // expert quarters (64 experts each)
-constexpr int RQ_NT = 256;                       // 4 waves; wave w owns expert tile 4*quarter + w
+constexpr int RQ_ET = E_GLOBAL / 16;             // expert tiles of 16, one per wave
+constexpr int ROUTER_CUS = 256;                  // the chip's CUs
 constexpr int RQ_NR = 4;                         // register ring depth (K-blocks)
 constexpr int RQ_KS = BLK / 32;                  // MFMA K steps per 128-column block
 constexpr int RQ_FRAG = 1024;                    // one 16 x 32 bf16 operand fragment
@@ -113,7 +114,7 @@ __device__ __forceinline__ float quot(float x, float s, float y) {
 }
 
 // The K loop's memory operations are inline assembly in a fixed order (per
-// K-block: the code store, then the 8 loads of the block three ahead)
+// K-block: the code store, then the loads of the block three ahead)
 // waited for with explicit counts: the compiler's own waits, merged
 // at the loop head across the unrolled ring and the loop's stores, drained
 // every load there.  The registers of a block pass through an empty asm
@@ -150,42 +151,53 @@ __device__ __forceinline__ uint32_t bslot(int tt, int ks, int g, int i) {
   return (uint32_t)(((tt * RQ_KS + ks) * 64 + g * 16 + (i ^ (c & 7))) * 16);
 }
 
-// Workgroup (token tile, expert quarter eq, K part kp): K-blocks kp*kpb ..
+// What bounds it is a CU's vector-memory path: per K-block a workgroup loads
+// 16 KB of rows and 4 KB of weights per wave, so more waves per workgroup
+// re-read the rows fewer times (four times with 4 waves, twice with 8, once
+// with 16), stage them fewer times, and leave the weights' bytes unchanged.
+//
+// Workgroup (token tile, expert part eq, K part kp): K-blocks kp*kpb ..
 // kp*kpb + kpb - 1.  out = logits [T, 256] when n_kp == 1, else partial sums
 // [n_kp][T][256].  Tokens past T read row T-1 and store nothing.  Workgroup
 // p runs on XCD p % 8: token tile t's workgroups all have p % 8 == t % 8, so
-// the four expert quarters that read a token tile's rows share one L2 (dealt
+// the expert parts that read a token tile's rows share one L2 (dealt
 // round-robin, they would fetch every row into four L2s).  The grid rounds
 // the tile count up to a multiple of 8; workgroups past the last tile exit.
-__global__ void __launch_bounds__(RQ_NT)
+template <int WAVES>
+__global__ void __launch_bounds__(64 * WAVES)
 router_quant_kernel(const uint8_t* __restrict__ hidden, const uint8_t* __restrict__ wpk, int T, int n_kp,
                     float* __restrict__ out, uint8_t* __restrict__ hq, float* __restrict__ hs) {
   __shared__ __attribute__((aligned(16))) uint8_t s_b[2][4 * RQ_KS * RQ_FRAG];  // 2 x 16 KB
-  __shared__ float s_qs[HB][16];  // the quantised rows' scales, written out after the K loop
+  constexpr int NT = 64 * WAVES, EQ = RQ_ET / WAVES;  // threads, expert parts
+  constexpr int CH = RQ_TOK * BLK / 8 / NT;           // 16-byte chunks a thread gathers per K-block
+  constexpr int ROWS = NT / 16;                       // token rows the workgroup's threads span
+  static_assert(CH == EQ, "each expert part quantises one of the CH row groups");
+  constexpr int LPK = CH + RQ_KS;                     // loads per K-block
+  __shared__ float s_qs[HB][ROWS];  // the quantised rows' scales, written out after the K loop
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int q = blockIdx.x / XCDS, rem = q % (RQ_EQ * n_kp);
-  const int tile = (q / (RQ_EQ * n_kp)) * XCDS + blockIdx.x % XCDS, eq = rem / n_kp, kp = rem % n_kp;
+  const int q = blockIdx.x / XCDS, rem = q % (EQ * n_kp);
+  const int tile = (q / (EQ * n_kp)) * XCDS + blockIdx.x % XCDS, eq = rem / n_kp, kp = rem % n_kp;
   if (tile * RQ_TOK >= T) return;
   const int kpb = HB / n_kp, kb0 = kp * kpb;
   const int t0 = tile * RQ_TOK;
 
-  // This thread's 4 chunks of a 64-token x 128-column block: chunk i is
-  // token r = tid/16 + 16*((i + eq) % 4), columns 8*(tid%16) .. +8 (16 bytes
-  // of bf16).  Chunk 0 holds the 16 rows this workgroup quantises.
-  uint32_t goff[4], sslot[4];
+  // This thread's CH chunks of a 64-token x 128-column block: chunk i is
+  // token r = tid/16 + ROWS*((i + eq) % CH), columns 8*(tid%16) .. +8 (16
+  // bytes of bf16).  Chunk 0 holds the ROWS rows this workgroup quantises.
+  uint32_t goff[CH], sslot[CH];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int r = (tid >> 4) + 16 * ((i + eq) & 3), c = tid & 15;
+  for (int i = 0; i < CH; ++i) {
+    const int r = (tid >> 4) + ROWS * ((i + eq) & (CH - 1)), c = tid & 15;
     goff[i] = (uint32_t)min(t0 + r, T - 1) * (H * 2) + c * 16;
     sslot[i] = bslot(r >> 4, c >> 2, c & 3, r & 15);
   }
   // Row this thread quantises (its chunk 0), clamped to T-1.
-  const int qrow = min(t0 + 16 * eq + (tid >> 4), T - 1);
+  const int qrow = min(t0 + ROWS * eq + (tid >> 4), T - 1);
   uint32_t rslot[RQ_KS];  // this lane's fragment position for each K step (token tile 0)
 #pragma unroll
   for (int ks = 0; ks < RQ_KS; ++ks) rslot[ks] = bslot(0, ks, lane >> 4, lane & 15);
-  const uint8_t* wbase = wpk + (size_t)(eq * 4 + w) * RQ_FRAG;  // + lane*16 per lane
+  const uint8_t* wbase = wpk + (size_t)(eq * WAVES + w) * RQ_FRAG;  // + lane*16 per lane
   const uint32_t wvoff = lane * 16;
   const uint32_t qoff = (uint32_t)qrow * H + (tid & 15) * 8;
 
@@ -194,10 +206,10 @@ router_quant_kernel(const uint8_t* __restrict__ hidden, const uint8_t* __restric
 #pragma unroll
   for (int tt = 0; tt < 4; ++tt) acc[tt] = zero4;
 
-  u32x4 v[RQ_NR][4], a[RQ_NR][RQ_KS];
+  u32x4 v[RQ_NR][CH], a[RQ_NR][RQ_KS];
   auto load = [&](int kb, int sl) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) gload(v[sl][i], goff[i], hidden + (size_t)kb * (BLK * 2));
+    for (int i = 0; i < CH; ++i) gload(v[sl][i], goff[i], hidden + (size_t)kb * (BLK * 2));
 #pragma unroll
     for (int ks = 0; ks < RQ_KS; ++ks) gload(a[sl][ks], wvoff, wbase + (size_t)kb * ROUTER_KB_BYTES + ks * (16 * RQ_FRAG));
   };
@@ -223,9 +235,9 @@ router_quant_kernel(const uint8_t* __restrict__ hidden, const uint8_t* __restric
   };
   // One K-block: wait for its loads, quantise, stage, multiply the previous
   // block, issue the loads three blocks ahead.  Block kb's loads are older
-  // than exactly WAIT operations: 18 in steady state (two K-blocks of code
-  // store + 8 loads), 16 / 17 in the first two blocks (the prologue loads
-  // have no stores between them).
+  // than exactly WAIT operations: 2 * (LPK + 1) in steady state (two K-blocks
+  // of code store + loads), 2 * LPK and one more in the first two blocks (the
+  // prologue loads have no stores between them).
   int kq = 0;
   auto step = [&](auto sl_c, auto wait_c, auto prev_c) {
     constexpr int sl = decltype(sl_c)::value, WAIT = decltype(wait_c)::value;
@@ -234,11 +246,11 @@ router_quant_kernel(const uint8_t* __restrict__ hidden, const uint8_t* __restric
     const int kb = kb0 + kq + sl;
     wait_vm<WAIT>();
 #pragma unroll
-    for (int i = 0; i < 4; ++i) __asm__ volatile("" : "+v"(v[sl][i]));
+    for (int i = 0; i < CH; ++i) __asm__ volatile("" : "+v"(v[sl][i]));
 #pragma unroll
     for (int ks = 0; ks < RQ_KS; ++ks) __asm__ volatile("" : "+v"(a[sl][ks]));
     {
-      // FP8 quantisation of this workgroup's 16 rows of the block (chunk
+      // FP8 quantisation of this workgroup's ROWS rows of the block (chunk
       // 0): the 16 lanes of a token hold its 128 columns.  The code store is
       // unconditional, a fixed operation count for the waits above (rows
       // past T rewrite row T-1 with the same bytes: they read row T-1); the
@@ -262,40 +274,40 @@ router_quant_kernel(const uint8_t* __restrict__ hidden, const uint8_t* __restric
     }
     uint8_t* sb = s_b[sl & 1];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) *reinterpret_cast<u32x4*>(sb + sslot[i]) = v[sl][i];
+    for (int i = 0; i < CH; ++i) *reinterpret_cast<u32x4*>(sb + sslot[i]) = v[sl][i];
     if constexpr (PREV) mma(s_b[(sl + 1) & 1], a[ps]);
     load(min(kb + RQ_NR - 1, kb0 + kpb - 1), ps);  // branch-free; the tail re-reads
     __syncthreads();
   };
   using std::integral_constant;
   using std::true_type;
-  step(integral_constant<int, 0>{}, integral_constant<int, 16>{}, std::false_type{});
-  step(integral_constant<int, 1>{}, integral_constant<int, 17>{}, true_type{});
-  step(integral_constant<int, 2>{}, integral_constant<int, 18>{}, true_type{});
-  step(integral_constant<int, 3>{}, integral_constant<int, 18>{}, true_type{});
+  step(integral_constant<int, 0>{}, integral_constant<int, 2 * LPK>{}, std::false_type{});
+  step(integral_constant<int, 1>{}, integral_constant<int, 2 * LPK + 1>{}, true_type{});
+  step(integral_constant<int, 2>{}, integral_constant<int, 2 * LPK + 2>{}, true_type{});
+  step(integral_constant<int, 3>{}, integral_constant<int, 2 * LPK + 2>{}, true_type{});
 #pragma unroll 1
   for (kq = RQ_NR; kq < kpb; kq += RQ_NR) {
-    step(integral_constant<int, 0>{}, integral_constant<int, 18>{}, true_type{});
-    step(integral_constant<int, 1>{}, integral_constant<int, 18>{}, true_type{});
-    step(integral_constant<int, 2>{}, integral_constant<int, 18>{}, true_type{});
-    step(integral_constant<int, 3>{}, integral_constant<int, 18>{}, true_type{});
+    step(integral_constant<int, 0>{}, integral_constant<int, 2 * LPK + 2>{}, true_type{});
+    step(integral_constant<int, 1>{}, integral_constant<int, 2 * LPK + 2>{}, true_type{});
+    step(integral_constant<int, 2>{}, integral_constant<int, 2 * LPK + 2>{}, true_type{});
+    step(integral_constant<int, 3>{}, integral_constant<int, 2 * LPK + 2>{}, true_type{});
   }
   wait_vm_all();  // the dead tail loads land before the registers are reused
   // the last block (ring slot 3, LDS buffer 1: kpb is a multiple of 4),
   // staged before the last step's barrier
   mma(s_b[1], a[RQ_NR - 1]);
   __syncthreads();
-  // Scales of the 16 quantised rows, [kb][T] layout: 16 consecutive tokens per K-block.
-  for (int j = tid; j < kpb * 16; j += RQ_NT) {
-    const int t = t0 + 16 * eq + (j & 15);
-    if (t < T) hs[(size_t)(kb0 + (j >> 4)) * T + t] = s_qs[j >> 4][j & 15];
+  // Scales of the quantised rows, [kb][T] layout: ROWS consecutive tokens per K-block.
+  for (int j = tid; j < kpb * ROWS; j += NT) {
+    const int t = t0 + ROWS * eq + j % ROWS;
+    if (t < T) hs[(size_t)(kb0 + j / ROWS) * T + t] = s_qs[j / ROWS][j % ROWS];
   }
   // D layout: lane l holds experts 4*(l/16) .. +3 of token column l%16.
 #pragma unroll
   for (int tt = 0; tt < 4; ++tt) {
     const int t = t0 + tt * 16 + (lane & 15);
     if (t < T) {
-      const int e = (eq * 4 + w) * 16 + 4 * (lane >> 4);
+      const int e = (eq * WAVES + w) * 16 + 4 * (lane >> 4);
       *reinterpret_cast<float4*>(out + ((size_t)kp * T + t) * E_GLOBAL + e) =
           make_float4(acc[tt][0], acc[tt][1], acc[tt][2], acc[tt][3]);
     }
@@ -317,14 +329,14 @@ logits_reduce_kernel(const float4* __restrict__ part, int n_kp, int n4, float4* 
 
 }  // namespace
 
-// K parts per launch: the fewest that give at least 448 workgroups (about
+// K parts per launch: the fewest that give at least 448 workgroups of four waves (about
 // two per CU; the K loop's dependent steps leave one workgroup per CU short
 // of the HBM rate), each part a multiple of the ring depth in K-blocks.
 // Measured: T=4096 51.5 -> 42.7 us with 2 parts (512 workgroups) instead of
 // 1; more parts than that lose to the partial sums' traffic and reduction
 // (T=8192 with 2 parts: 77 -> 81 us; T=1024 with 14: 19.9 -> 25.5 us).
 int router_k_parts(int T) {
-  const int groups = RQ_EQ * ((T + RQ_TOK - 1) / RQ_TOK);
+  const int groups = 4 * ((T + RQ_TOK - 1) / RQ_TOK);
   const int parts[] = {1, 2, 7, 14};
   for (int p : parts)
     if (groups * p >= 448) return p;
@@ -352,9 +364,29 @@ hipError_t launch_router_quant(const uint8_t* hidden_bf16, const uint8_t* router
   if (T <= 0) return hipSuccess;
   const int n_kp = router_k_parts(T);
   const int tiles8 = ((T + RQ_TOK - 1) / RQ_TOK + XCDS - 1) / XCDS * XCDS;
-  const int grid = RQ_EQ * n_kp * tiles8;
-  router_quant_kernel<<<grid, RQ_NT, 0, stream>>>(hidden_bf16, router_packed, T, n_kp, n_kp > 1 ? partial : logits,
-                                                  hidden_fp8, hidden_scale);
+  auto launch = [&](auto kernel, int waves) {
+    kernel<<<RQ_ET / waves * n_kp * tiles8, 64 * waves, 0, stream>>>(
+        hidden_bf16, router_packed, T, n_kp, n_kp > 1 ? partial : logits, hidden_fp8, hidden_scale);
+  };
+  // One workgroup of 16 or 8 waves runs per CU, so these are taken where they
+  // fill 7/10 of their rounds of the chip's CUs, or 9/10 of several rounds
+  // over the whole K range, whose last one is long; parts of a single ring
+  // (14 K parts, small T) stay with four waves, which spread over more CUs.
+  // Same K parts, 4 / 8 / 16 waves: T=2048 30.1 / 28.1 / 24.2 us, T=3300 46.4
+  // / 48.0 / 39.7, T=4096 36.5 / 34.3 / 41.0, T=6000 50.0 / 54.5 / 45.3,
+  // T=8192 60 / 53 / 68, T=11000 99.6 / 115.5 / 100.2, T=13000 124 / 120 / 105,
+  // T=16384 138 / 129 / 116, T=20000 172 / 181 / 196, T=24000 202 / 192 / 208.
+  auto fills = [&](int groups) {
+    const int rounds = (groups + ROUTER_CUS - 1) / ROUTER_CUS;
+    return 10 * groups >= (n_kp == 1 && rounds > 1 ? 9 : 7) * rounds * ROUTER_CUS;
+  };
+  const int tiles = (T + RQ_TOK - 1) / RQ_TOK;
+  if (n_kp < 14 && fills(tiles * n_kp))
+    launch(router_quant_kernel<16>, 16);
+  else if (n_kp < 14 && fills(2 * tiles * n_kp))
+    launch(router_quant_kernel<8>, 8);
+  else
+    launch(router_quant_kernel<4>, 4);
   hipError_t err = hipGetLastError();
   if (err != hipSuccess || n_kp == 1) return err;
   const int n4 = T * E_GLOBAL / 4;

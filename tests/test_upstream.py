@@ -212,6 +212,27 @@ def test_router_quant_full_size_sampled(ops, cuda, router):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("T", [2017, 3585, 3649, 7151, 11649])
+def test_router_quant_wide_workgroups(ops, cuda, router, T):
+    """Sizes whose workgroups have 16 waves (2017: seven K parts, 11649: one)
+    and 8 (3585 and 3649: two parts, 7151: one), each with a ragged last
+    token tile; rows at the tile edges, and every row's codes and scales."""
+    w, packed = router
+    bits = _hidden_bits(T, 40 + T)
+    logits, hq, hs = ops.router_quant(_to_dev(bits, cuda), packed)
+    torch.cuda.synchronize()
+    print(f"router_quant wide T={T}", flush=True)
+    codes, scale = up.act_quant(bits)
+    assert np.array_equal(hq.view(torch.uint8).cpu().numpy(), codes)
+    assert np.array_equal(hs.cpu().numpy(), scale)
+    rows = np.unique(np.r_[0:80, 127:130, T // 2:T // 2 + 64, T - 70:T])
+    exact = up.router_logits(bits[rows], w)
+    err = np.abs(logits.cpu().numpy()[rows].astype(np.float64) - exact)
+    assert (err <= LOGIT_REL * up.logits_bound(bits[rows], w) + 1e-30).all()
+    assert torch.equal(ops.router_quant(_to_dev(bits, cuda), packed)[0], logits)
+
+
+@pytest.mark.gpu
 def test_router_quant_feeds_forward(ops, inputs_mod, cuda, router):
     """The produced tensors are moe_forward inputs: the forward over them
     equals, bit for bit, the forward over the oracle's codes and scales with

@@ -43,9 +43,12 @@ def _stream(device: torch.device) -> ctypes.c_void_p:
 
 
 def _require_device(name: str, t: torch.Tensor, device: torch.device | None = None) -> None:
-    _check(t.is_cuda, f"{name} must be a HIP device tensor (no CPU path)")
-    if device is not None:
-        _check(t.device == device, f"{name} must be on {device}, got {t.device}")
+    # The messages are formatted only for the error: eighteen of them on every
+    # forward cost more host time than the launches of a one-token call.
+    if not t.is_cuda:
+        raise RuntimeError(f"{name} must be a HIP device tensor (no CPU path)")
+    if device is not None and t.device != device:
+        raise RuntimeError(f"{name} must be on {device}, got {t.device}")
 
 
 # --------------------------------------------------------------------------- packs
@@ -200,12 +203,15 @@ def _validate_forward(hidden, hidden_scale, W13_packed, W13_scale, W2_packed, W2
     _check(W2_packed.size(0) == E and tuple(W2_packed.shape[1:]) == W2_PACKED_SHAPE,
            "W2_packed must be [E_local, 56, 16, 8, 2, 64, 4]")
     _check(tuple(W2_scale.shape) == (E, H_BLOCKS, I_BLOCKS), "W2_scale must be [E_local, 56, 16]")
-    _check(1 <= E <= MAX_E_LOCAL, f"E_local must be in [1, {MAX_E_LOCAL}], got {E}")
+    if not 1 <= E <= MAX_E_LOCAL:
+        raise RuntimeError(f"E_local must be in [1, {MAX_E_LOCAL}], got {E}")
+    dev = hidden.device
     for name, t in (("hidden", hidden), ("hidden_scale", hidden_scale), ("W13_packed", W13_packed),
                     ("W13_scale", W13_scale), ("W2_packed", W2_packed), ("W2_scale", W2_scale),
                     ("logits", logits), ("bias", bias)):
-        _check(t.is_contiguous(), f"{name} must be contiguous")
-        _require_device(name, t, hidden.device)
+        if not t.is_contiguous():
+            raise RuntimeError(f"{name} must be contiguous")
+        _require_device(name, t, dev)
     return T, E
 
 

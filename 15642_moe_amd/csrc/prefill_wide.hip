@@ -47,25 +47,24 @@ struct WideGeom {
 };
 
 // Direct global -> LDS loads: lane l's 16 (4) bytes at sbase + voff land at
-// LDS address lds + 16 l (4 l).  M0 holds the LDS address; the kernels use it
-// for nothing else.  They are counted by vmcnt like any load, and the
-// compiler knows nothing of them: every wait is explicit (landed_barrier,
-// wait_loads).  The wait states in front also cover a base address that a
-// VALU instruction has just written (the reload of a spilled scalar register;
-// five states to its use by a memory instruction, which the compiler does not
-// insert for inline assembly).  NTL: non-temporal.
+// LDS address lds + 16 l (4 l).  M0 holds the LDS address.  It is an operand
+// that the compiler writes: it uses M0 too (as the lane select of v_writelane,
+// in the wave reduction around the queue's atomics).  The loads are counted by
+// vmcnt like any other, and the compiler knows nothing of them: every wait is
+// explicit (landed_barrier, wait_loads).  The wait states in front cover M0's
+// write and a base address that a VALU instruction has just written (the
+// reload of a spilled scalar register; five states to its use by a memory
+// instruction, which the compiler does not insert for inline assembly).
+// NTL: non-temporal.
 template <bool NTL>
 __device__ __forceinline__ void dma16(uint32_t lds, uint32_t voff, const void* sbase) {
   if constexpr (NTL)
-    __asm__ volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tglobal_load_lds_dwordx4 %1, %2 nt" ::"s"(lds), "v"(voff), "s"(sbase)
-                     : "memory");
+    __asm__ volatile("s_nop 4\n\tglobal_load_lds_dwordx4 %1, %2 nt" ::"{m0}"(lds), "v"(voff), "s"(sbase) : "memory");
   else
-    __asm__ volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(voff), "s"(sbase)
-                     : "memory");
+    __asm__ volatile("s_nop 4\n\tglobal_load_lds_dwordx4 %1, %2" ::"{m0}"(lds), "v"(voff), "s"(sbase) : "memory");
 }
 __device__ __forceinline__ void dma4(uint32_t lds, uint32_t voff, const void* sbase) {
-  __asm__ volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tglobal_load_lds_dword %1, %2" ::"s"(lds), "v"(voff), "s"(sbase)
-                   : "memory");
+  __asm__ volatile("s_nop 4\n\tglobal_load_lds_dword %1, %2" ::"{m0}"(lds), "v"(voff), "s"(sbase) : "memory");
 }
 // All but this wave's N youngest loads have landed and its LDS reads are done;
 // then all waves meet.

@@ -7,6 +7,10 @@ reads it.  The compiler inserts them for its own instructions and not for
 those inside inline assembly, so a reload right before such a load gives it a
 stale base address.  Every kernel that issues vector-memory instructions
 from inline assembly is checked on every path of its control flow.
+
+M0, the LDS address of a global -> LDS load, must reach such a load as an
+operand that the compiler writes: the compiler uses M0 itself, and does not
+know of a write inside inline assembly.
 """
 
 from __future__ import annotations
@@ -107,3 +111,27 @@ def test_checker_flags_a_reload_before_a_load():
     assert not check_scalar_operands(["v_readlane_b32 s6, v221, 15", *load])
     assert not check_scalar_operands(["v_readlane_b32 s4, v221, 15", "s_mov_b32 s4, 0", *load])
     assert check_scalar_operands(["v_readlane_b32 s4, v221, 15", "s_cbranch_scc1 .LBB0_2", "s_endpgm", ".LBB0_2:", *load])
+
+
+def asm_writes_of_m0(lines: list[str]) -> list[str]:
+    """Instructions inside inline assembly whose destination is M0."""
+    in_asm, found = False, []
+    for raw in lines:
+        if ";;#ASMSTART" in raw or ";;#ASMEND" in raw:
+            in_asm = ";;#ASMSTART" in raw
+            continue
+        _, _, rest = raw.split(";")[0].strip().partition(" ")
+        if in_asm and rest.split(",")[0].strip() == "m0":
+            found.append(raw.strip())
+    return found
+
+
+@pytest.mark.skipif(not HIPCC, reason="hipcc not available")
+def test_inline_assembly_leaves_m0_to_the_compiler():
+    lds_loads = 0
+    for name, lines in _kernels(_device_asm("prefill_wide.hip")):
+        assert not asm_writes_of_m0(lines), f"{name} writes M0 in inline assembly"
+        lds_loads += sum("global_load_lds" in line for line in lines)
+    assert lds_loads > 0
+    assert asm_writes_of_m0([";;#ASMSTART", "s_mov_b32 m0, s4", ";;#ASMEND"])
+    assert not asm_writes_of_m0(["s_mov_b32 m0, s4", ";;#ASMSTART", "s_nop 4", "global_load_lds_dword v1, s[2:3]", ";;#ASMEND"])

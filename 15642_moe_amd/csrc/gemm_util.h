@@ -2,8 +2,7 @@
 #pragma once
 
 #include "common.h"
-
-#include <mutex>
+#include "launch.h"
 
 namespace moe {
 
@@ -185,22 +184,6 @@ __device__ __forceinline__ void tile_routes(int e, int mt, const int* s_tp, cons
 // ---------------------------------------------------------------------------
 // Host side.
 // ---------------------------------------------------------------------------
-
-// Compute units of the current device (cached per device).
-inline int device_cus() {
-  static std::mutex mu;
-  static int cus_of[64] = {0};
-  int dev = 0;
-  (void)hipGetDevice(&dev);
-  std::lock_guard<std::mutex> lk(mu);
-  int& c = cus_of[dev & 63];
-  if (c == 0) {
-    int cus = 0;
-    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) cus = 256;
-    c = cus;
-  }
-  return c;
-}
 
 template <typename K>
 int resident_blocks(K kernel, int threads) {

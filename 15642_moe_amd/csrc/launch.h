@@ -4,7 +4,25 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <mutex>
+
 namespace moe {
+
+// Compute units of the current device (cached per device).
+inline int device_cus() {
+  static std::mutex mu;
+  static int cus_of[64] = {0};
+  int dev = 0;
+  (void)hipGetDevice(&dev);
+  std::lock_guard<std::mutex> lk(mu);
+  int& c = cus_of[dev & 63];
+  if (c == 0) {
+    int cus = 0;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) cus = 256;
+    c = cus;
+  }
+  return c;
+}
 
 // `queue` (may be null) = the MOE_WS_QUEUE buffer: its work-queue counters
 // and, where launch_dispatch needs them zero, its per-chunk counts are
@@ -65,7 +83,6 @@ hipError_t launch_stage2_decode(const uint8_t* Cq, const float* Cs, const uint8_
 
 // Producer of the forward's inputs (router logits + FP8 activations) from
 // bf16 hidden states; `partial` holds router_partial_bytes(T) (unused when 0).
-int router_k_parts(int T);
 size_t router_partial_bytes(int T);
 hipError_t launch_pack_router(const uint8_t* w, uint8_t* packed, bool unpack, hipStream_t stream);
 hipError_t launch_router_quant(const uint8_t* hidden_bf16, const uint8_t* router_packed, int T, float* partial,

@@ -34,9 +34,6 @@ namespace {
 
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 
-constexpr int RQ_TOK = 64;                       // tokens per workgroup (4 tiles of 16)
-constexpr int RQ_ET = E_GLOBAL / 16;             // expert tiles of 16, one per wave
-constexpr int ROUTER_CUS = 256;                  // the chip's CUs
 constexpr int RQ_NR = 4;                         // register ring depth (K-blocks)
 constexpr int RQ_KS = BLK / 32;                  // MFMA K steps per 128-column block
 constexpr int RQ_FRAG = 1024;                    // one 16 x 32 bf16 operand fragment
@@ -329,20 +326,6 @@ logits_reduce_kernel(const float4* __restrict__ part, int n_kp, int n4, float4* 
 
 }  // namespace
 
-// K parts per launch: the fewest that give at least 448 workgroups of four waves (about
-// two per CU; the K loop's dependent steps leave one workgroup per CU short
-// of the HBM rate), each part a multiple of the ring depth in K-blocks.
-// Measured: T=4096 51.5 -> 42.7 us with 2 parts (512 workgroups) instead of
-// 1; more parts than that lose to the partial sums' traffic and reduction
-// (T=8192 with 2 parts: 77 -> 81 us; T=1024 with 14: 19.9 -> 25.5 us).
-int router_k_parts(int T) {
-  const int groups = 4 * ((T + RQ_TOK - 1) / RQ_TOK);
-  const int parts[] = {1, 2, 7, 14};
-  for (int p : parts)
-    if (groups * p >= 448) return p;
-  return 14;
-}
-
 size_t router_partial_bytes(int T) {
   const int p = router_k_parts(T);
   return p > 1 ? (size_t)p * T * E_GLOBAL * sizeof(float) : 0;
@@ -368,22 +351,10 @@ hipError_t launch_router_quant(const uint8_t* hidden_bf16, const uint8_t* router
     kernel<<<RQ_ET / waves * n_kp * tiles8, 64 * waves, 0, stream>>>(
         hidden_bf16, router_packed, T, n_kp, n_kp > 1 ? partial : logits, hidden_fp8, hidden_scale);
   };
-  // One workgroup of 16 or 8 waves runs per CU, so these are taken where they
-  // fill 7/10 of their rounds of the chip's CUs, or 9/10 of several rounds
-  // over the whole K range, whose last one is long; parts of a single ring
-  // (14 K parts, small T) stay with four waves, which spread over more CUs.
-  // Same K parts, 4 / 8 / 16 waves: T=2048 30.1 / 28.1 / 24.2 us, T=3300 46.4
-  // / 48.0 / 39.7, T=4096 36.5 / 34.3 / 41.0, T=6000 50.0 / 54.5 / 45.3,
-  // T=8192 60 / 53 / 68, T=11000 99.6 / 115.5 / 100.2, T=13000 124 / 120 / 105,
-  // T=16384 138 / 129 / 116, T=20000 172 / 181 / 196, T=24000 202 / 192 / 208.
-  auto fills = [&](int groups) {
-    const int rounds = (groups + ROUTER_CUS - 1) / ROUTER_CUS;
-    return 10 * groups >= (n_kp == 1 && rounds > 1 ? 9 : 7) * rounds * ROUTER_CUS;
-  };
-  const int tiles = (T + RQ_TOK - 1) / RQ_TOK;
-  if (n_kp < 14 && fills(tiles * n_kp))
+  const int waves = router_waves(T, device_cus());
+  if (waves == 16)
     launch(router_quant_kernel<16>, 16);
-  else if (n_kp < 14 && fills(2 * tiles * n_kp))
+  else if (waves == 8)
     launch(router_quant_kernel<8>, 8);
   else
     launch(router_quant_kernel<4>, 4);

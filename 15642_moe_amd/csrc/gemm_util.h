@@ -114,7 +114,6 @@ __device__ __forceinline__ void load_tile_table(const int32_t* __restrict__ coun
 // weight block to the next.  Measured by FETCH_SIZE at skewed T=4096 (four
 // experts of 4096 routes): GEMM1 moved 3.0x its algorithmic bytes in plain
 // (weight block, route tile) order.
-constexpr int WORK_BAND = 8;
 __device__ __forceinline__ void decode_work(int L, int nblk, int e_local, const int* s_tp, int& e, int& blk,
                                             int& mt) {
   const int l = threadIdx.x & 63, li = l < e_local ? l : 0;  // every read inside s_tp[0 .. e_local]

@@ -4,6 +4,12 @@
 // this file by itself.
 #pragma once
 
+#ifdef __HIPCC__
+#define MOE_HD __host__ __device__ __forceinline__
+#else
+#define MOE_HD inline
+#endif
+
 namespace moe {
 
 constexpr int H = 7168;            // hidden size
@@ -74,6 +80,68 @@ inline int router_waves(int T, int cus) {
     if (10 * groups >= tenths * rounds * xcd_cus) return waves;
   }
   return 4;
+}
+
+// ---------------------------------------------------------------------------
+// Work lists of the wide prefill GEMMs (prefill_wide.hip): which tile size a
+// launch takes, which items an XCD's queue holds and in which order.
+// ---------------------------------------------------------------------------
+constexpr int WORK_BAND = 8;  // route tiles of a band (see decode_work in gemm_util.h)
+
+// A launch's tile sizes, in 32-route fragments, and an item's cost by its
+// fragments, of which only the ratio matters: what a K-block of an item takes
+// beside its fragments (weights, barriers, LDS latency) is worth about 8
+// fragments where most items of a launch have few of them.
+// The launch's length is estimated as whole rounds of items over the
+// workgroups x the mean item, and the least one's size is taken; sizes 3 and 2
+// only where tiles of 4 leave some workgroup without an item, since cutting
+// finer only then puts idle CUs to work.  Over 1000 launches (16 to 32 local
+// experts, T = 3072 .. 16384, even, uneven and skewed routing) the choice takes
+// 1.0% more than the best of the five sizes in the mean and 6% in the worst
+// 20th; with sizes 3 and 2 always open 1.2% and 7% (even routing, T=3300 with
+// 18 experts: 5% slower than the kernels of prefill.hip instead of equal).
+// An estimate from the items' sum, max(largest item, sum / CUs + half an item),
+// is 2.8 to 3.7% off for GEMM1, with these costs or with a full tile's clocks.
+constexpr int TILE_SIZES = 5, TILE_COARSE = 3;  // the first TILE_COARSE are always open
+constexpr int TILE_FRAGS[TILE_SIZES] = {8, 6, 4, 3, 2};
+constexpr float ITEM_COST = 1500.0f, FRAG_COST = 190.0f;
+
+MOE_HD int route_frags(int routes) { return (routes + 31) >> 5; }
+MOE_HD int route_tiles(int frags, int tile_frags) { return (frags + tile_frags - 1) / tile_frags; }
+// First route of tile mt (0 .. nt) of an expert with f fragments in nt tiles:
+// the fragments are dealt evenly.
+MOE_HD int tile_first_route(int mt, int f, int nt) { return 32 * ((mt * f) / nt); }
+
+// A launch of `tiles` route tiles with `frags` fragments in all, each x nblk
+// weight blocks, over `workgroups`.
+MOE_HD float launch_estimate(int tiles, int frags, int nblk, int workgroups) {
+  const int rounds = (tiles * nblk + workgroups - 1) / workgroups;
+  return (float)rounds * (ITEM_COST + FRAG_COST * ((float)frags / (float)(tiles > 0 ? tiles : 1)));
+}
+// Index into TILE_FRAGS; `fine`: tiles of 4 give at most one item per workgroup.
+MOE_HD int pick_tile(const float* est, bool fine) {
+  int best = 0;
+  for (int i = 1; i < TILE_SIZES; ++i)
+    if ((i < TILE_COARSE || fine) && est[i] < est[best]) best = i;
+  return best;
+}
+
+// Order of the experts: by fragments per item (key), descending.
+MOE_HD bool expert_before(int key_a, int a, int key_b, int b) { return key_a > key_b || (key_a == key_b && a < b); }
+// Place in the order of the i-th expert of queue x: descending in the even
+// queues, ascending in the odd ones.
+MOE_HD int order_place(int x, int i) { return x & 1 ? MAX_E_LOCAL - 1 - i : i; }
+// Items of queue x from the expert at place p of the order, which has nt route
+// tiles and U quads of weight blocks: quad j is queue (U * p + j) % XCDS's.
+MOE_HD int queue_items(int x, int U, int p, int nt) { return ((x - U * p) & (XCDS - 1)) < U ? 4 * nt : 0; }
+// Weight block and route tile of the local-th of them: bands of WORK_BAND
+// route tiles, then weight block, then route tile.
+MOE_HD void queue_item(int x, int U, int p, int nt, int local, int& blk, int& mt) {
+  const int full = nt / WORK_BAND, b = local / (4 * WORK_BAND), band = b < full ? b : full;
+  const int width = b < full ? WORK_BAND : nt - full * WORK_BAND;
+  const int r = local - band * 4 * WORK_BAND;
+  blk = 4 * ((x - U * p) & (XCDS - 1)) + r / width;
+  mt = band * WORK_BAND + r % width;
 }
 
 }  // namespace moe

@@ -133,9 +133,11 @@ __device__ __forceinline__ void wait_loads() { __asm__ volatile("s_waitcnt vmcnt
 // Work distribution.  A launch's items are (local expert, weight block of 256
 // rows, route tile); WideWork lists them per XCD queue.
 //
+// The arithmetic is plan.h's, which a CPU test compiles.
+//
 // Tile size: each expert's 32-route fragments are dealt evenly over
-// ceil(fragments / tile) route tiles, with one tile size per launch, the one of
-// TILE_FRAGS with the least rounds x mean item cost: a few experts with many
+// ceil(fragments / tile) route tiles, with one tile size per launch, chosen
+// from TILE_FRAGS by the launch's estimated length: a few experts with many
 // routes are cut finer where whole tiles would leave CUs without an item.
 // Order: experts by fragments per item, descending in the even queues and
 // ascending in the odd ones: items of few routes stream weights from HBM and
@@ -149,17 +151,12 @@ __device__ __forceinline__ void wait_loads() { __asm__ volatile("s_waitcnt vmcnt
 // a time: what one fetch into its L2 serves.  Within a quad: bands of
 // WORK_BAND route tiles, then weight block, then route tile.
 // ---------------------------------------------------------------------------
-constexpr int TILE_FRAGS[5] = {8, 6, 4, 3, 2};
-constexpr float ITEM_COST = 1500.0f, FRAG_COST = 190.0f;  // clocks per K-block of an item: fixed, per fragment
-
-// Place in the order of the i-th expert of queue x.
-__device__ __forceinline__ int order_place(int x, int i) { return x & 1 ? MAX_E_LOCAL - 1 - i : i; }
-
 struct WideWork {
   int ord[MAX_E_LOCAL];                   // the expert at each place of the order
   int cnt[MAX_E_LOCAL], off[MAX_E_LOCAL], nt[MAX_E_LOCAL];  // per expert: routes, first route, route tiles
   int first[XCDS][MAX_E_LOCAL + 1];       // first[x][i]: items of queue x before its i-th expert's
-  float est[8];
+  float est[TILE_SIZES];                  // the launch's estimated length with each tile size
+  int fine;                               // sizes below 4 fragments are open
 };
 
 __device__ __forceinline__ int sum32(int v) {
@@ -172,29 +169,25 @@ template <int NBLK, int U>
 __device__ __forceinline__ void build_work(WideWork& wk, const int32_t* __restrict__ counts,
                                            const int32_t* __restrict__ offsets, int e_local) {
   static_assert(NBLK == 4 * U && U <= XCDS, "quads");
-  constexpr int NT = 5;
+  static_assert(TILE_SIZES <= WNT / 64 && TILE_FRAGS[TILE_COARSE - 1] == 4, "one tile size per wave");
   const int e = threadIdx.x & 31, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int c = e < e_local ? counts[e] : 0, o = e < e_local ? offsets[e] : 0;
-  const int f = (c + 31) >> 5;
-  if (wave < NT) {
-    const int k = TILE_FRAGS[wave];
-    const int tiles = sum32((f + k - 1) / k), frags = sum32(f);
-    const int rounds = (tiles * NBLK + (int)gridDim.x - 1) / (int)gridDim.x;
-    if (threadIdx.x % 64 == 0)
-      wk.est[wave] = (float)rounds * (ITEM_COST + FRAG_COST * ((float)frags / (float)max(tiles, 1)));
+  const int f = route_frags(c);
+  if (wave < TILE_SIZES) {
+    const int tiles = sum32(route_tiles(f, TILE_FRAGS[wave])), frags = sum32(f);
+    if (threadIdx.x % 64 == 0) {
+      wk.est[wave] = launch_estimate(tiles, frags, NBLK, (int)gridDim.x);
+      if (wave == TILE_COARSE - 1) wk.fine = tiles * NBLK <= (int)gridDim.x;
+    }
   }
   __syncthreads();
-  int best = 0;
-#pragma unroll
-  for (int i = 1; i < NT; ++i) best = wk.est[i] < wk.est[best] ? i : best;
-  const int k = TILE_FRAGS[best];
+  const int k = TILE_FRAGS[pick_tile(wk.est, wk.fine)];
   if (threadIdx.x < MAX_E_LOCAL) {
-    const int nt = (f + k - 1) / k, key = nt ? (f + nt - 1) / nt : 0;
+    const int nt = route_tiles(f, k), key = nt ? route_tiles(f, nt) : 0;
     int rank = 0;
 #pragma unroll
     for (int j = 0; j < MAX_E_LOCAL; ++j) {
-      const int kj = __builtin_amdgcn_readlane(key, j);
-      rank += (kj > key || (kj == key && j < e)) ? 1 : 0;
+      rank += expert_before(__builtin_amdgcn_readlane(key, j), j, key, e) ? 1 : 0;
     }
     wk.ord[rank] = e;
     wk.cnt[e] = c;
@@ -204,7 +197,7 @@ __device__ __forceinline__ void build_work(WideWork& wk, const int32_t* __restri
   __syncthreads();
   if (threadIdx.x < XCDS * MAX_E_LOCAL) {
     const int x = threadIdx.x >> 5, i = e, p = order_place(x, i);
-    int inc = ((x - U * p) & (XCDS - 1)) < U ? 4 * wk.nt[wk.ord[p]] : 0;
+    int inc = queue_items(x, U, p, wk.nt[wk.ord[p]]);
 #pragma unroll
     for (int d = 1; d < 32; d <<= 1) {
       const int y = __shfl_up(inc, d, 32);
@@ -225,11 +218,7 @@ __device__ __forceinline__ void work_item(const WideWork& wk, int x, int idx, in
   e = __builtin_amdgcn_readfirstlane(wk.ord[p]);
   const int nt = __builtin_amdgcn_readfirstlane(wk.nt[e]);
   const int local = idx - __builtin_amdgcn_readfirstlane(wk.first[x][i]);
-  const int full = nt / WORK_BAND, band = local / (4 * WORK_BAND);
-  const int width = band < full ? WORK_BAND : nt - full * WORK_BAND;
-  const int r = local - min(band, full) * 4 * WORK_BAND;
-  blk = 4 * ((x - U * p) & (XCDS - 1)) + r / width;
-  mt = min(band, full) * WORK_BAND + r % width;
+  queue_item(x, U, p, nt, local, blk, mt);
 }
 
 // Claims of a persistent workgroup (wave 0's lane 0): its own XCD's queue
@@ -326,8 +315,8 @@ wide_kernel(const uint8_t* __restrict__ act, const float* __restrict__ ascale, c
     mt = __builtin_amdgcn_readfirstlane(mt);
     // fragments [mt * f / nt, (mt + 1) * f / nt) of the expert's f
     const int cnt = __builtin_amdgcn_readfirstlane(wk.cnt[e]), nt = __builtin_amdgcn_readfirstlane(wk.nt[e]);
-    const int f = (cnt + 31) >> 5, m0 = 32 * ((mt * f) / nt);
-    it.rows = min(cnt, 32 * (((mt + 1) * f) / nt)) - m0;
+    const int f = route_frags(cnt), m0 = tile_first_route(mt, f, nt);
+    it.rows = min(cnt, tile_first_route(mt + 1, f, nt)) - m0;
     it.rb = __builtin_amdgcn_readfirstlane(wk.off[e]) + m0;
     const int ncc = (it.rows + RT - 1) / RT, nc0 = (ncc + 1) >> 1;
     it.ncw = wc ? ncc - nc0 : nc0;

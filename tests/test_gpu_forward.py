@@ -524,6 +524,45 @@ def test_forward_wide_prefill_tiles(ops, cuda, T, e_local, hot):
     assert torch.equal(out.view(torch.int16), out2.view(torch.int16))
 
 
+@pytest.mark.parametrize("routes,gemm1,gemm2", [
+    ({5: 1024}, 2, 4), ({0: 1500}, 3, 6), ({15: 1024, 3: 480}, 3, 6), ({7: 2048}, 4, 8), ({2: 3072}, 6, 6),
+    ({5: 512}, 2, 2), ({15: 750}, 2, 3), ({}, 8, 8)])
+def test_forward_wide_prefill_tile_sizes(ops, cuda, tmp_path, routes, gemm1, gemm2):
+    """The wide prefill GEMMs with each of their tile sizes (few busy experts
+    are cut finer) and without any local route: T=3300 and 16 local experts,
+    the first `n` tokens of `routes` on an expert each, all other picks
+    outside the rank."""
+    from conftest import pkg
+    from test_plan import build_plan, wide_tile
+
+    layer = pkg("moe_layer")
+    T, e_local = 3300, 16
+    inp = layer.build_moe_inputs(T=T, device="cuda", seed=T + len(routes))
+    for k in ("gemm1_weights", "gemm1_weights_scale", "gemm2_weights", "gemm2_weights_scale"):
+        inp[k] = inp[k][:e_local].contiguous()
+    logits = torch.randn(T, 256, generator=torch.Generator().manual_seed(T)) - 12.0
+    logits[:, 224:] += 20.0
+    logits[:, :e_local] -= 40.0
+    for e, n in routes.items():
+        logits[:n, e] += 80.0
+    inp["routing_logits"] = logits.to("cuda")
+    r = ops.route(inp["routing_logits"], inp["routing_bias"].float(), 1.0, int(inp["local_expert_offset"]), e_local)
+    counts = r["counts"].cpu().tolist()
+    assert counts == [routes.get(e, 0) for e in range(e_local)]
+    plan, cus = build_plan(tmp_path), torch.cuda.get_device_properties(0).multi_processor_count
+    if cus == 256:
+        assert (wide_tile(plan, counts, 16), wide_tile(plan, counts, 28)) == (gemm1, gemm2)
+    print(f"[forward] wide tile sizes {routes}", flush=True)
+    out = layer.run_custom(ops, **inp)
+    out2 = layer.run_custom(ops, **inp)
+    torch.cuda.synchronize()
+    if routes:
+        _check_against_models(f"wide tile sizes {routes}", out, _cpu(inp))
+    else:
+        assert not out.any()
+    assert torch.equal(out.view(torch.int16), out2.view(torch.int16))
+
+
 @pytest.mark.parametrize("case", range(6))
 def test_forward_random_shapes(ops, cuda, case):
     """Seeded random (T, local_expert_offset, E_local, routed_scaling_factor)

@@ -8,6 +8,7 @@ import shutil
 import subprocess
 from pathlib import Path
 
+import numpy as np
 import pytest
 
 from conftest import REPO
@@ -23,6 +24,11 @@ def build_plan(out_dir: Path) -> ctypes.CDLL:
     subprocess.run([gxx, "-O1", "-std=c++17", "-Wall", "-Werror", "-shared", "-fPIC", f"-I{CSRC}",
                     str(REPO / "tests" / "plan_host.cpp"), "-o", str(so)], check=True)
     return ctypes.CDLL(str(so))
+
+
+def wide_tile(plan, counts, nblk, workgroups=256) -> int:
+    """The tile size, in 32-route fragments, of a wide prefill GEMM (nblk 16: GEMM1, 28: GEMM2)."""
+    return plan.plan_wide_tile((ctypes.c_int * len(counts))(*counts), len(counts), nblk, workgroups)
 
 
 @pytest.fixture(scope="module")
@@ -52,3 +58,49 @@ def test_router_waves_fill_their_rounds(plan, cus):
         groups = 16 // waves * -(-(-(-T // 64)) // 8) * parts
         if waves > 4:
             assert groups >= 0.7 * per_xcd * -(-groups // per_xcd)
+
+
+@pytest.mark.parametrize("counts,gemm1,gemm2", [
+    ([0] * 16, 8, 8),
+    # one busy expert: cut as fine as there are workgroups for
+    ([512] + [0] * 15, 2, 2), ([768] + [0] * 15, 2, 3), ([1024] + [0] * 15, 2, 4), ([1536] + [0] * 15, 3, 6),
+    ([2048] + [0] * 15, 4, 8), ([3072] + [0] * 15, 6, 6),
+    # more items than workgroups with tiles of four fragments: no finer, though three and two fill the last round
+    ([96] * 10 + [128] * 10, 8, 8), ([105] * 18, 8, 8),
+    ([128] * 32, 8, 8), ([288] * 12 + [256] * 4, 6, 6)])
+def test_wide_tile_size(plan, counts, gemm1, gemm2):
+    assert (wide_tile(plan, counts, 16), wide_tile(plan, counts, 28)) == (gemm1, gemm2)
+
+
+@pytest.mark.parametrize("seed", range(24))
+def test_wide_items_cover_every_tile_once(plan, seed):
+    """The items of the kernels' own arithmetic: for any route counts, each
+    (expert, weight block) has its routes dealt to items once, in whole
+    fragments, and none holds more than the tile size; an expert's blocks lie
+    in quads on different queues."""
+    rng = np.random.default_rng(seed)
+    e_local = int(rng.integers(1, 33))
+    counts = [int(c) for c in rng.choice([0, 1, 31, 32, 33, 255, 256, 257, 513, 2304, 2305, 4096], size=e_local)]
+    for nblk in (16, 28):
+        for tile in {8, 6, 4, 3, 2, wide_tile(plan, counts, nblk)}:
+            room = 2 * nblk * (sum(counts) // 32 + 33)
+            buf = np.zeros((room, 5), dtype=np.int32)
+            n = plan.plan_wide_items((ctypes.c_int * e_local)(*counts), e_local, nblk, tile,
+                                     buf.ctypes.data_as(ctypes.POINTER(ctypes.c_int)), room)
+            assert n >= 0
+            spans: dict = {}
+            for x, e, blk, first, rows in buf[:n].tolist():
+                assert 0 <= e < e_local and 0 <= blk < nblk and 0 < rows <= 32 * tile and first % 32 == 0
+                spans.setdefault((e, blk), []).append((first, rows, x))
+            assert set(spans) == {(e, b) for e in range(e_local) if counts[e] for b in range(nblk)}
+            for (e, blk), got in spans.items():
+                at = 0
+                for first, rows, x in sorted(got):
+                    assert first == at and x == got[0][2]
+                    at += rows
+                assert at == counts[e]
+            for e in range(e_local):
+                if counts[e]:
+                    queue_of = [spans[e, 4 * j][0][2] for j in range(nblk // 4)]
+                    assert len(set(queue_of)) == nblk // 4
+                    assert all(spans[e, b][0][2] == queue_of[b // 4] for b in range(nblk))

@@ -774,23 +774,13 @@ hipError_t run_stage2_tile(const uint8_t* Cq, const float* Cs, const uint8_t* w2
   return hipGetLastError();
 }
 
-// Large batches take the 256 x 256-tile kernels of prefill_wide.hip: from 96
-// expected routes per local expert (T / 32) on, and with at least 16 local
-// experts.  Measured, wide against these kernels (whole forward): even routing
-// T=2048 315 / 304 us, 2500 319 / 311, 3500 344 / 344, 4096 358 / 418, 6000 413 /
-// 494; uneven T=1500 269 / 257, 3001 331 / 338; with 16 local experts T=5000
-// 220 / 221 and T=16384 512 / 546.  With 8 local experts a 256-row item per
-// weight block leaves CUs without work unless the routing is skewed: T=4096
-// 163 / 143, T=8192 207 / 199, skewed T=4096 835 / 936.
-bool wide_path(int T, int e_local) { return T >= 3072 && e_local >= 16; }
-
 }  // namespace
 
 hipError_t launch_stage1(const uint8_t* hidden, const float* hidden_scale, const uint8_t* w13p,
                          const float* w13_scale, const int32_t* counts, const int32_t* offsets,
                          const int32_t* route_token, uint8_t* Cq, float* Cs, int T, int e_local, int max_routes,
                          int32_t* queue, hipStream_t stream) {
-  if (wide_path(T, e_local))
+  if (prefill_wide(T, e_local, device_cus()))
     return launch_stage1_wide(hidden, hidden_scale, w13p, w13_scale, counts, offsets, route_token, Cq, Cs, T, e_local,
                               max_routes, queue, stream);
   if (!stage1_wide_tiles(T))
@@ -805,7 +795,7 @@ hipError_t launch_stage2(const uint8_t* Cq, const float* Cs, const uint8_t* w2p,
                          const int32_t* route_token, float* Y, uint16_t* out,
                          int T, int e_local, int max_routes, int32_t* queue,
                          hipStream_t stream) {
-  if (wide_path(T, e_local))
+  if (prefill_wide(T, e_local, device_cus()))
     return launch_stage2_wide(Cq, Cs, w2p, w2_scale, counts, offsets, route_weight, route_token, Y, out, T, e_local,
                               max_routes, queue, stream);
   if (stage2_narrow_tiles(T))

@@ -60,6 +60,15 @@ def test_router_waves_fill_their_rounds(plan, cus):
             assert groups >= 0.7 * per_xcd * -(-groups // per_xcd)
 
 
+@pytest.mark.parametrize("T,e_local,wide", [
+    (3071, 32, 0), (3072, 32, 1), (3071, 17, 0), (3072, 17, 1), (3072, 16, 0), (3150, 16, 0), (3199, 16, 0),
+    (3200, 16, 1), (16384, 16, 1), (3200, 15, 0), (16384, 8, 0), (129, 32, 0)])
+def test_prefill_wide_on_256_cus(plan, T, e_local, wide):
+    """The wide kernels' line: later where an item per weight block is at most
+    one per CU."""
+    assert plan.plan_prefill_wide(T, e_local, 256) == wide
+
+
 @pytest.mark.parametrize("counts,gemm1,gemm2", [
     ([0] * 16, 8, 8),
     # one busy expert: cut as fine as there are workgroups for

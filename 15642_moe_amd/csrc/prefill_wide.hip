@@ -55,16 +55,22 @@ struct WideGeom {
 // write and a base address that a VALU instruction has just written (the
 // reload of a spilled scalar register; five states to its use by a memory
 // instruction, which the compiler does not insert for inline assembly).
-// NTL: non-temporal.
-template <bool NTL>
+// NTL: non-temporal.  K, which the assembly carries as a comment: what the load
+// brings, by which a test follows the counted waits.
+enum LoadKind { K_WEIGHTS, K_ACTIVATIONS, K_TABLES };
+template <bool NTL, LoadKind K>
 __device__ __forceinline__ void dma16(uint32_t lds, uint32_t voff, const void* sbase) {
   if constexpr (NTL)
-    __asm__ volatile("s_nop 4\n\tglobal_load_lds_dwordx4 %1, %2 nt" ::"{m0}"(lds), "v"(voff), "s"(sbase) : "memory");
+    __asm__ volatile("s_nop 4\n\tglobal_load_lds_dwordx4 %1, %2 nt ; kind %3"
+                     ::"{m0}"(lds), "v"(voff), "s"(sbase), "n"(K) : "memory");
   else
-    __asm__ volatile("s_nop 4\n\tglobal_load_lds_dwordx4 %1, %2" ::"{m0}"(lds), "v"(voff), "s"(sbase) : "memory");
+    __asm__ volatile("s_nop 4\n\tglobal_load_lds_dwordx4 %1, %2 ; kind %3"
+                     ::"{m0}"(lds), "v"(voff), "s"(sbase), "n"(K) : "memory");
 }
+template <LoadKind K>
 __device__ __forceinline__ void dma4(uint32_t lds, uint32_t voff, const void* sbase) {
-  __asm__ volatile("s_nop 4\n\tglobal_load_lds_dword %1, %2" ::"{m0}"(lds), "v"(voff), "s"(sbase) : "memory");
+  __asm__ volatile("s_nop 4\n\tglobal_load_lds_dword %1, %2 ; kind %3"
+                   ::"{m0}"(lds), "v"(voff), "s"(sbase), "n"(K) : "memory");
 }
 // All but this wave's N youngest loads have landed and its LDS reads are done;
 // then all waves meet.
@@ -335,8 +341,8 @@ wide_kernel(const uint8_t* __restrict__ act, const float* __restrict__ ascale, c
   auto issue_w1 = [&](const WideItem& it, uint32_t alane, int kb, int slot, int i) __attribute__((always_inline)) {
     const uint8_t* p = it.wsrc + (size_t)kb * WKB + (i >> 1) * 512 + (i & 1) * 1024;
     const uint32_t d = lw + slot * W_SLOT + op_w * FRAG + i * 1024;
-    if (it.nt) dma16<true>(d, alane, p);
-    else dma16<false>(d, alane, p);
+    if (it.nt) dma16<true, K_WEIGHTS>(d, alane, p);
+    else dma16<false, K_WEIGHTS>(d, alane, p);
   };
   auto issue_w = [&](const WideItem& it, int kb, int slot) __attribute__((always_inline)) {
     const uint32_t alane = a_lane_offset(fresh_lane());
@@ -344,11 +350,11 @@ wide_kernel(const uint8_t* __restrict__ act, const float* __restrict__ ascale, c
     for (int i = 0; i < 4; ++i) issue_w1(it, alane, kb, slot, i);
   };
   auto issue_a1 = [&](const WideItem& it, int kb, int slot, int i) __attribute__((always_inline)) {
-    dma16<false>(la + slot * G::ACT_SLOT + (it.tile0 + i) * FRAG + wr * 1024, aoff[i], act + (size_t)kb * BLK);
+    dma16<false, K_ACTIVATIONS>(la + slot * G::ACT_SLOT + (it.tile0 + i) * FRAG + wr * 1024, aoff[i], act + (size_t)kb * BLK);
   };
   // 64 lanes: the 32 scales of one of the wave's route tiles, twice
   auto issue_s = [&](const WideItem& it, int kb, int slot) __attribute__((always_inline)) {
-    dma4(ls + slot * (G::SCL_SLOT * 4) + (it.tile0 + min(wr, it.ncw - 1)) * 256, soff,
+    dma4<K_ACTIVATIONS>(ls + slot * (G::SCL_SLOT * 4) + (it.tile0 + min(wr, it.ncw - 1)) * 256, soff,
          S1 ? ascale + (size_t)kb * T : ascale + kb);
   };
   // The item's tables, one load per wave: route tokens (waves 0-3), stage 2's
@@ -358,12 +364,12 @@ wide_kernel(const uint8_t* __restrict__ act, const float* __restrict__ ascale, c
     const int r = 64 * wr + lane;
     const uint32_t off = (uint32_t)(it.rb + (r < it.rows ? r : 0)) * 4u;
     if (wc == 0) {
-      dma4(lds_addr(&s_rt[par][0][64 * wr]), off, route_token);
+      dma4<K_TABLES>(lds_addr(&s_rt[par][0][64 * wr]), off, route_token);
     } else if constexpr (!S1) {
-      dma4(lds_addr(&s_rt[par][1][64 * wr]), off, route_weight);
+      dma4<K_TABLES>(lds_addr(&s_rt[par][1][64 * wr]), off, route_weight);
     }
     if (wc == 1 && wr < 2)  // gate / up blocks nb, IB + nb; H blocks 2nb, 2nb + 1
-      dma4(lds_addr(&s_ws[par][wr][0]), it.sofs + (uint32_t)(wr * (S1 ? IB * HB : IB) + min(lane, KB - 1)) * 4u, wscale);
+      dma4<K_TABLES>(lds_addr(&s_ws[par][wr][0]), it.sofs + (uint32_t)(wr * (S1 ? IB * HB : IB) + min(lane, KB - 1)) * 4u, wscale);
   };
   // Per-lane row offsets of an item's activations and scales (stage 1: its
   // route tokens are in s_rt[par][0]).  Activation chunks: lane = route

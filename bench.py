@@ -7,7 +7,7 @@
 A step is one moe_forward (route, dispatch, GEMM1+SwiGLU+FP8 requant,
 GEMM2, combine) over one batch with pre-packed weights already resident in
 HBM; the one-time pack is timed separately.  The headline line is the decode
-configuration (T=64, BASELINE configs[1]); the other configurations are timed
+configuration (T=64); the other configurations are timed
 too and reported under "configs".  Per-kernel durations come from HIP events
 recorded on the launch stream between the kernels (moe_forward_timed), and
 give the roofline figure of the dominant kernel.  Each configuration is also
@@ -32,9 +32,11 @@ from __future__ import annotations
 
 import argparse
 import ctypes
+import hashlib
 import importlib
 import json
 import os
+import re
 import sys
 import time
 from pathlib import Path
@@ -52,23 +54,32 @@ def log(msg: str) -> None:
     print(f"[bench] {msg}", file=sys.stderr, flush=True)
 
 
-def _traffic_from_profiles(config_name: str) -> dict:
+def _kernel_sources_hash(csrc: Path = REPO / "15642_moe_amd" / "csrc") -> str:
+    """Hash of the kernel sources without comments and white space."""
+    h = hashlib.sha256()
+    for p in sorted([*csrc.glob("*.hip"), *csrc.glob("*.h")]):
+        h.update(p.name.encode())
+        h.update(re.sub(r"\s+", "", re.sub(r"//.*", "", p.read_text())).encode())
+    return h.hexdigest()[:16]
+
+
+def _traffic_from_profiles(config_name: str, profiles: Path = REPO / "profiles") -> dict:
     """HBM bytes per launch of the dominant kernel, the kernel and the commit
     it was measured at, from the committed rocprofv3 PMC summary
     (profiles/traffic_<workload>.txt: 'traffic_bytes_per_launch: N',
-    'dominant_kernel: ...', 'commit: ...'); values None when absent."""
+    'dominant_kernel: ...', 'commit: ...', 'sources: ...'); values None when
+    absent, or when the kernels have changed since (the summary's 'sources' is
+    not the hash of those here)."""
     rec = {"traffic": None, "traffic_kernel": None, "traffic_commit": None}
-    p = REPO / "profiles" / f"traffic_{config_name}.txt"
+    p = profiles / f"traffic_{config_name}.txt"
     if not p.exists():
         return rec
-    for line in p.read_text().splitlines():
-        key, _, val = line.partition(":")
-        if key == "traffic_bytes_per_launch":
-            rec["traffic"] = float(val)
-        elif key == "dominant_kernel":
-            rec["traffic_kernel"] = val.strip()
-        elif key == "commit":
-            rec["traffic_commit"] = val.strip()
+    found = {key: val.strip() for key, _, val in (line.partition(":") for line in p.read_text().splitlines())}
+    if found.get("sources") != _kernel_sources_hash():
+        return rec
+    rec["traffic"] = float(found["traffic_bytes_per_launch"])
+    rec["traffic_kernel"] = found.get("dominant_kernel")
+    rec["traffic_commit"] = found.get("commit")
     return rec
 
 
@@ -298,9 +309,9 @@ def main() -> int:
         "scaling": "weak",
         "vs_baseline": None,
         "dtype": "fp8_e4m3",
-        "data": "synthetic: counter-based generator, BASELINE distributions (N(0,1) e4m3 weights/activations)",
+        "data": "synthetic: counter-based generator, N(0,1) e4m3 weights and activations, uniform scales",
         "config": {
-            "workload": "decode_T64 (BASELINE configs[1]): DeepSeek-V3 MoE layer, T=64, H=7168, I=2048, "
+            "workload": "decode_T64: DeepSeek-V3 MoE layer, T=64, H=7168, I=2048, "
                         "256 experts / 32 local (offset 0), top-8 of 8 groups (top-4 groups), rsf 2.5",
             "T": 64,
             "local_routes": head["local_routes"],

@@ -532,9 +532,6 @@ hipError_t launch_mfma_ceiling(float* out, unsigned long long* clocks, int iters
 // ---------------------------------------------------------------------------
 // Host launchers.
 // ---------------------------------------------------------------------------
-// The most local experts that T tokens can hit.
-static int decode_experts(int T, int e_local) { return T * TOP_K < e_local ? T * TOP_K : e_local; }
-
 hipError_t launch_stage1_decode(const int32_t* topk_ids, const float* topk_w, int T, int e_local, int offset,
                                 const uint8_t* hidden, const float* hidden_scale, const uint8_t* w13p,
                                 const float* w13_scale, int32_t* counts, int32_t* offsets, int32_t* route_token,
@@ -575,12 +572,16 @@ hipError_t launch_stage2_decode(const uint8_t* Cq, const float* Cs, const uint8_
   // An expert holds at most T routes: one fragment up to 16 tokens, two per
   // weight pass above (skewed T=30 106 -> 99 us for the whole call, skewed
   // T=64 261 -> 245; even T=32 79.8 -> 81.2).
-  if (T > 16)
-    stage2_decode_kernel<4, 2, 4><<<grid, 256, 0, stream>>>(Cq, Cs, w2p, w2_scale, counts, offsets, route_weight,
-                                                            route_token, Y, out, e_local);
+  auto launch = [&](auto kernel, int kw) {
+    kernel<<<grid, 64 * kw, 0, stream>>>(Cq, Cs, w2p, w2_scale, counts, offsets, route_weight, route_token, Y, out,
+                                         e_local);
+  };
+  if (stage2_decode_waves(T, e_local, device_cus()) == 1)
+    launch(stage2_decode_kernel<4, 2, 1>, 1);
+  else if (T > 16)
+    launch(stage2_decode_kernel<4, 2, 4>, 4);
   else
-    stage2_decode_kernel<4, 1, 4><<<grid, 256, 0, stream>>>(Cq, Cs, w2p, w2_scale, counts, offsets, route_weight,
-                                                            route_token, Y, out, e_local);
+    launch(stage2_decode_kernel<4, 1, 4>, 4);
   return hipGetLastError();
 }
 

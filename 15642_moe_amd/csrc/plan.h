@@ -82,6 +82,25 @@ inline int router_waves(int T, int cus) {
   return 4;
 }
 
+// The most local experts that T tokens can hit.
+inline int decode_experts(int T, int e_local) { return T * TOP_K < e_local ? T * TOP_K : e_local; }
+
+// Waves that share the K range of a decode GEMM2 item (expert, 64 weight rows):
+// four, so that an item has more loads in flight; one above 64 tokens where
+// the items nearly fill the chip and are all resident at once as single waves
+// (two per SIMD: more than 6 and at most 8 per CU, 14 to 18 local experts), which
+// four-wave workgroups, two per CU, need 3.1 to 3.9 rounds for.  Whole call,
+// weights not in cache, four waves / one, us: even routing, 16 local experts T=72
+// 122.3 / 119.3, T=128 128.5 / 125.2 (and the next call's GEMM1 with it), 14 T=96
+// 117.5 / 114.6, 18 T=96 145.7 / 144.2; uneven, 16 T=128 86.3 / 87.1; skewed,
+// 16 T=128 220 / 230 (231 before the split).  Outside: 12, even T=128 99.0 /
+// 99.0, 19 149.6 / 151.5, 32 231.9 / 239.1; 16, even T=48 115.1 / 114.3, T=64
+// 119.2 / 118.8.
+inline int stage2_decode_waves(int T, int e_local, int cus) {
+  const int items = decode_experts(T, e_local) * (H / 64);
+  return T > 64 && items > 6 * cus && items <= 8 * cus ? 1 : 4;
+}
+
 // Whether both prefill GEMMs of T tokens run in the 256 x 256-tile kernels of
 // prefill_wide.hip: with at least 16 local experts, from T = 3072 on (96 expected
 // routes per expert), or 3200 where an item per weight block is at most one per

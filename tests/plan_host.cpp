@@ -6,6 +6,7 @@ extern "C" {
 int plan_router_k_parts(int T) { return moe::router_k_parts(T); }
 int plan_router_waves(int T, int cus) { return moe::router_waves(T, cus); }
 
+int plan_stage2_decode_waves(int T, int e_local, int cus) { return moe::stage2_decode_waves(T, e_local, cus); }
 int plan_prefill_wide(int T, int e_local, int cus) { return moe::prefill_wide(T, e_local, cus); }
 
 // The tile size (fragments) that a wide prefill GEMM with nblk weight blocks per expert takes.

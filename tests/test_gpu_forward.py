@@ -475,6 +475,30 @@ def test_forward_decode_items(ops, cuda, T, e_local, experts):
     assert torch.equal(out.view(torch.int16), out2.view(torch.int16))
 
 
+@pytest.mark.parametrize("T,e_local,hot", [(64, 16, 0), (65, 16, 0), (128, 16, 0), (96, 14, 3), (128, 18, 7), (128, 13, 0)])
+def test_forward_decode_single_wave_items(ops, cuda, T, e_local, hot):
+    """Decode GEMM2 items of one wave (14 to 18 local experts above 64 tokens)
+    and the sizes beside them: every local expert hit by some token, `hot` of
+    them by every token (several passes over their weights)."""
+    from conftest import pkg
+
+    layer = pkg("moe_layer")
+    inp = layer.build_moe_inputs(T=T, device="cuda", seed=T + e_local)
+    for k in ("gemm1_weights", "gemm1_weights_scale", "gemm2_weights", "gemm2_weights_scale"):
+        inp[k] = inp[k][:e_local].contiguous()
+    logits = torch.randn(T, 256, generator=torch.Generator().manual_seed(T)) - 12.0
+    logits[:, 224:] += 20.0  # every token's remaining picks, outside the local experts
+    logits[torch.arange(T), torch.arange(T) % e_local] += 40.0
+    logits[:, :hot] += 40.0
+    inp["routing_logits"] = logits.to("cuda")
+    print(f"[forward] decode single-wave items T={T} E_local={e_local} hot={hot}", flush=True)
+    out = layer.run_custom(ops, **inp)
+    out2 = layer.run_custom(ops, **inp)
+    torch.cuda.synchronize()
+    _check_against_models(f"decode single-wave items T={T} E={e_local}", out, _cpu(inp))
+    assert torch.equal(out.view(torch.int16), out2.view(torch.int16))
+
+
 @pytest.mark.parametrize("T", [1024, 1025])
 def test_forward_skewed_either_side_of_the_gemm2_tile_switch(ops, cuda, T):
     """Routing bias +3 on local experts 0-3 (as config 4) at T = 1024 (GEMM2

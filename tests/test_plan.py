@@ -60,6 +60,15 @@ def test_router_waves_fill_their_rounds(plan, cus):
             assert groups >= 0.7 * per_xcd * -(-groups // per_xcd)
 
 
+@pytest.mark.parametrize("T,e_local,waves", [
+    (1, 32, 4), (64, 16, 4), (65, 16, 1), (128, 16, 1), (65, 13, 4), (65, 14, 1), (128, 18, 1), (128, 19, 4),
+    (128, 32, 4), (128, 8, 4), (2, 16, 4)])
+def test_stage2_decode_waves_on_256_cus(plan, T, e_local, waves):
+    """One wave per decode GEMM2 item where the items fill one round of single
+    waves: more than 6 and at most 8 per CU."""
+    assert plan.plan_stage2_decode_waves(T, e_local, 256) == waves
+
+
 @pytest.mark.parametrize("T,e_local,wide", [
     (3071, 32, 0), (3072, 32, 1), (3071, 17, 0), (3072, 17, 1), (3072, 16, 0), (3150, 16, 0), (3199, 16, 0),
     (3200, 16, 1), (16384, 16, 1), (3200, 15, 0), (16384, 8, 0), (129, 32, 0)])

@@ -1,10 +1,39 @@
 // Shared definitions for the MI355X (gfx950) FP8 MoE forward kernels.
+//
+// Geometry is the fixed DeepSeek-V3/R1 routed-expert layer used by the
+// reference (kernels/moe.cu:41-53, reference/moe_ref.py:27-46).  It is all that
+// a plain C++ compiler sees of this file (the CPU tests of plan.h).
 #pragma once
+
+namespace moe {
+
+constexpr int H = 7168;            // hidden size
+constexpr int I = 2048;            // expert intermediate size
+constexpr int G1 = 2 * I;          // W13 rows (gate rows 0..I-1, up rows I..2I-1)
+constexpr int E_GLOBAL = 256;
+constexpr int N_GROUP = 8;
+constexpr int GROUP_SIZE = E_GLOBAL / N_GROUP;  // 32
+constexpr int TOP_K = 8;
+constexpr int TOPK_GROUP = 4;
+constexpr int BLK = 128;           // scale block along every K/N axis
+constexpr int HB = H / BLK;        // 56 hidden blocks
+constexpr int IB = I / BLK;        // 16 intermediate blocks
+constexpr int G1B = G1 / BLK;      // 32 W13 row blocks
+constexpr int MAX_E_LOCAL = 32;    // dispatch uses a 32-bit local-expert mask per token
+constexpr float E4M3_MAX = 448.0f;
+// Largest token count served by the decode kernels (dispatch fused into GEMM1).
+constexpr int DECODE_MAX_T = 128;
+// Work-queue words of the prefill GEMMs, for each of the two: a claim
+// counter per XCD, then a mask of the XCD segments found drained.
+constexpr int XCDS = 8;
+constexpr int QUEUE_COUNTERS = 2 * (XCDS + 1);
+
+}  // namespace moe
+
+#ifdef __HIPCC__
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
-
-#include "plan.h"
 
 namespace moe {
 
@@ -117,3 +146,5 @@ __host__ __device__ __forceinline__ uint64_t mix64(uint64_t z) {
 constexpr uint64_t GOLDEN = 0x9E3779B97F4A7C15ull;
 
 }  // namespace moe
+
+#endif  // __HIPCC__

@@ -3,6 +3,7 @@
 
 #include "common.h"
 #include "launch.h"
+#include "plan.h"
 
 namespace moe {
 

@@ -26,6 +26,7 @@
 // deterministic.
 #include "common.h"
 #include "launch.h"
+#include "plan.h"
 
 #include <type_traits>
 

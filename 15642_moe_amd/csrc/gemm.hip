@@ -32,17 +32,19 @@ namespace moe {
 // and no barrier in the K loop.  Where items are few or short, KW waves of a
 // workgroup take a part of the item's K-blocks each and the first adds the
 // parts in K order: more loads in flight per item, and a part that fits the
-// ring has all of them in flight at once.  GEMM2's 16 K-blocks by four waves,
-// whole call: T=64 uneven 136 -> 135 us, T=96 224 -> 215, T=113 even 225 ->
-// 217, skewed T=128 323 -> 308.
+// ring has all of them in flight at once.  GEMM2's 16 K-blocks by four waves
+// (its time, weights not in cache, even routing over 32 local experts): T=4
+// 16.8 -> 13.9 us, T=32 59.8 -> 54.3, T=113 85.7 -> 79.5, skewed T=128 132 -> 116.
 // Items are dealt expert-major over the experts that have routes, found from
 // the picks (GEMM1) or counts (GEMM2) by every workgroup; since workgroup p
 // runs on XCD p % 8, every expert's slices are dealt round-robin over all
 // XCDs.  The grid holds the experts that T tokens can hit at most, and
-// workgroups past the hit ones exit at once.  (With a static grid over all
-// experts and a 32-step count loop in each workgroup the empty ones cost as
-// much as the streaming at small T: T=4 54 -> 41 us, T=8 73 -> 60, T=16
-// 70 -> 55, T=32 90 -> 80 without them.)
+// workgroups past the hit ones exit at once.  (A static grid over all experts
+// and a 32-step count loop in each workgroup cost as much as the streaming at
+// small T.  Whole call with both this and the K split, weights not in cache,
+// even routing over 32 local experts: T=4 52 -> 40 us, T=8 83 -> 71, T=16 125 ->
+// 108, T=32 178 -> 162, T=64 218 -> 210, T=113 237 -> 230; 16 local experts that
+// are all hit, T=96..128, 125 -> 127.)
 // ---------------------------------------------------------------------------
 
 // Lane k's value of v (k wave-uniform): the weight-block scales sit one
@@ -550,7 +552,10 @@ hipError_t launch_stage1_decode(const int32_t* topk_ids, const float* topk_w, in
   // 133.6; T=64 even 185.0 and 181.0, uneven 133.0 and 130.8).  Above, hot
   // experts hold several fragments: two per weight pass and two pairs per
   // wave (skewed T=90 263 us, where one fragment and one pair take 321;
-  // even T=113 218 and 213).
+  // even T=113 218 and 213).  Up to 64 two fragments would shorten skewed
+  // routing (T=30 99.5 -> 87.3, T=64 251 -> 223) and lengthen uneven routing
+  // (T=37 88.8 -> 99.6).  (One batch back to back, its weights partly in the
+  // Infinity Cache.)
   if (T > 64)
     launch(stage1_decode_kernel<4, 2, 2, 1>, 2, 1);
   else if (T > 32)
@@ -571,7 +576,7 @@ hipError_t launch_stage2_decode(const uint8_t* Cq, const float* Cs, const uint8_
   const int grid = decode_experts(T, e_local) * (H / 64);
   // An expert holds at most T routes: one fragment up to 16 tokens, two per
   // weight pass above (skewed T=30 106 -> 99 us for the whole call, skewed
-  // T=64 261 -> 245; even T=32 79.8 -> 81.2).
+  // T=64 266 -> 251; even T=32 79.8 -> 81.2; one batch back to back).
   auto launch = [&](auto kernel, int kw) {
     kernel<<<grid, 64 * kw, 0, stream>>>(Cq, Cs, w2p, w2_scale, counts, offsets, route_weight, route_token, Y, out,
                                          e_local);

@@ -11,19 +11,24 @@
 // operands per 16.8 MFLOP K-block step, where the register-staged 256 x 192
 // tile moves 56 KB per 12.6.
 //
-// What a step is bound by (skewed T=4096, clocks per K-block of a full tile; the
-// MFMA pipe alone needs 2048): 2640 without any loads -- the two barriers and
-// the weight fragments' LDS latency, ~400, and 280-290 per route tile where the
-// pipe needs 256 -- and 2640-2840 with them.  The instruction order inside a
-// route tile matters more than anything else (below); all loads at the
-// step's start instead of one behind each MFMA cost 540 clocks.  At this
-// density the chip lowers its clock (2.2 -> 1.9 GHz), which takes back about
-// half of what the step gains.
+// What a step is bound by.  The MFMA pipe alone needs 2048 clocks per K-block of
+// a full tile.  Timing copies at skewed T=4096, before the wait states in front
+// of the loads (dma16), took 2640 without any loads -- the two barriers and the
+// weight fragments' LDS latency, ~400, and 280-290 per route tile where the pipe
+// needs 256 -- and 2640-2840 with them.  The instruction order inside a route
+// tile matters more than anything else (below); all loads at the step's start
+// instead of one behind each MFMA cost 540 clocks.  Over whole launches, where
+// most tiles are partial, the counters point to the operands' arrival: at T=8192
+// the pipe is busy 44% (GEMM1) and 35% (GEMM2) of the cycles, the waves wait 42%
+// and 48% of theirs, and the L1 is stalled ~40% on L2 data; GEMM1 moves 1.37 GB
+// from beyond L2 (1.7x its algorithmic bytes) at 4.7 TB/s.  At full density the chip lowers
+// its clock (2.2 -> 1.7-1.9 GHz), which takes back about half of what the step
+// gains.  The wait states cost 1 to 5% of GEMM1.
 //
 // Measured against the register-staged kernels on the same box (GEMM1 / GEMM2
-// us): T=16384 even routing 572 / 328 -> 485 / 318, T=8192 uneven 319 / 178 ->
-// 267 / 174, skewed T=4096 618 / 374 -> 493 / 347, T=4096 even 241 / 125 -> 182
-// / 127.
+// us): T=16384 even routing 557 / 342 -> 500 / 328, T=8192 uneven 314 / 179 ->
+// 290 / 179, skewed T=4096 623 / 381 -> 519 / 355, T=4096 even 248 / 137 -> 198
+// / 132.
 #include "common.h"
 #include "gemm_util.h"
 #include "launch.h"
@@ -154,7 +159,9 @@ __device__ __forceinline__ void wait_loads() { __asm__ volatile("s_waitcnt vmcnt
 // of the expert at place p belongs to XCD (U * p + j) % 8, so an expert's quads lie
 // on different XCDs and each XCD has at most one of them (U <= 8), holds a
 // share of every cost class, and runs 4 weight blocks x up to 8 route tiles at
-// a time: what one fetch into its L2 serves.  Within a quad: bands of
+// a time, which share their fetches into its L2 as far as they stay in step
+// (skewed T=4096: GEMM1 moves 1.9x its algorithmic bytes, the register-staged
+// kernels 2.0x; T=8192: 1.7x and 1.5x).  Within a quad: bands of
 // WORK_BAND route tiles, then weight block, then route tile.
 // ---------------------------------------------------------------------------
 struct WideWork {
@@ -261,7 +268,7 @@ struct WideQueue {
 // operand's of the previous route tile, then the first operand's of this one.
 // Two product buffers suffice, no FMA waits for the MFMA right before it, and
 // the pipe always holds the next MFMA.  With all of a product's 16 FMAs in one
-// place between MFMAs a full tile's step took 3600 clocks, in this order 2880.
+// place between MFMAs a full tile's step took a quarter longer.
 //
 // Between items: the next item is claimed during the last two steps; its
 // tables, first weights and (stage 2) activations are loaded under the

@@ -520,8 +520,8 @@ def test_forward_skewed_either_side_of_the_gemm2_tile_switch(ops, cuda, T):
 
 @pytest.mark.parametrize("T,e_local,hot", [(3071, 32, 0), (3072, 32, 0), (3072, 16, 0), (3333, 17, 3), (3100, 31, 9)])
 def test_forward_wide_prefill_tiles(ops, cuda, T, e_local, hot):
-    """The wide prefill GEMMs (T >= 3072 and 16 or more local experts) and
-    the last T below them.  hot > 0: exact route counts at the edges of
+    """The wide prefill GEMMs (T >= 3072 and more than 16 local experts; with
+    16, T >= 3200) and sizes just below them.  hot > 0: exact route counts at the edges of
     fragments, tiles and bands on the first experts (each token's other
     picks are spread over the rest), so that some experts have 0, 1, 32, 33,
     256, 257 and more than eight tiles' worth of routes."""

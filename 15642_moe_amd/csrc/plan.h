@@ -82,24 +82,26 @@ inline int stage2_decode_waves(int T, int e_local, int cus) {
 
 // Whether both prefill GEMMs of T tokens run in the 256 x 256-tile kernels of
 // prefill_wide.hip: with at least 16 local experts, from T = 3072 on (96 expected
-// routes per expert), or 3200 where an item per weight block is at most one per
-// CU: such a launch is a single round, in which a wide item takes longer to
-// stream its weights, and routes past the 96th cost the kernels of prefill.hip
-// a fragment more.  Whole forward, weights not in cache, prefill.hip / wide, us:
+// routes per expert), or 3456 (108) where an item per weight block is at most one
+// per CU: such a launch is a single round of the kernels of prefill.hip too, as
+// long as no expert has more than 128 routes (108 and twice the deviation of
+// even routing), and a wide item takes longer to stream its weights.
+// Whole forward, weights not in cache, prefill.hip / wide, us:
 //   32 local experts, even  T=2800 306 / 316, 3072 319 / 322, 3200 333 / 325, 3500
 //     368 / 330, 4096 418 / 347, 8192 576 / 542, 16384 996 / 909
 //     uneven 2500 / 3072 / 4096 / 8192: 0.96, 0.97, 0.95, 0.93 of prefill.hip's
 //     time; skewed 3072 885 / 812, 4096 1098 / 985
 //   24, even   3072 262 / 267, 3500 271 / 273, 4096 331 / 283; uneven 3072 297 / 281
 //   17, even   3072 224 / 226, 3500 227 / 229, 5000 270 / 259; uneven 3072 219 / 220
-//   16, even   3072 175 / 185, 3150 177 / 189, 3200 186 / 189, 3300 185 / 191, 3500
-//     196 / 192, 4096 236 / 196, 4500 201 / 201, 8192 317 / 314; uneven 3150 197 /
-//     194, 3300 206 / 198; skewed 3150 800 / 740, 3200 799 / 740
+//   16, even   3072 175 / 185, 3231 177 / 188, 3341 176 / 189, 3474 189 / 192, 3526
+//     215 / 194, 4096 236 / 196, 4329 195 / 199, 4910 206 / 206, 5500 252 / 222, 8192
+//     317 / 314; uneven 3176 190 / 186, 3326 218 / 207, 3561 232 / 220; skewed 3335
+//     848 / 780
 // With 8 local experts a 256-row item per weight block leaves CUs without work
 // unless the routing is skewed: T=4096 143 / 163, T=8192 199 / 207, skewed
 // T=4096 936 / 835.
 inline bool prefill_wide(int T, int e_local, int cus) {
-  return e_local >= 16 && T >= (e_local * IB <= cus ? 3200 : 3072);
+  return e_local >= 16 && T >= (e_local * IB <= cus ? 3456 : 3072);
 }
 
 // ---------------------------------------------------------------------------

@@ -521,7 +521,7 @@ def test_forward_skewed_either_side_of_the_gemm2_tile_switch(ops, cuda, T):
 @pytest.mark.parametrize("T,e_local,hot", [(3071, 32, 0), (3072, 32, 0), (3072, 16, 0), (3333, 17, 3), (3100, 31, 9)])
 def test_forward_wide_prefill_tiles(ops, cuda, T, e_local, hot):
     """The wide prefill GEMMs (T >= 3072 and more than 16 local experts; with
-    16, T >= 3200) and sizes just below them.  hot > 0: exact route counts at the edges of
+    16, T >= 3456) and sizes just below them.  hot > 0: exact route counts at the edges of
     fragments, tiles and bands on the first experts (each token's other
     picks are spread over the rest), so that some experts have 0, 1, 32, 33,
     256, 257 and more than eight tiles' worth of routes."""
@@ -553,14 +553,14 @@ def test_forward_wide_prefill_tiles(ops, cuda, T, e_local, hot):
     ({5: 512}, 2, 2), ({15: 750}, 2, 3), ({}, 8, 8)])
 def test_forward_wide_prefill_tile_sizes(ops, cuda, tmp_path, routes, gemm1, gemm2):
     """The wide prefill GEMMs with each of their tile sizes (few busy experts
-    are cut finer) and without any local route: T=3300 and 16 local experts,
+    are cut finer) and without any local route: T=3456 and 16 local experts,
     the first `n` tokens of `routes` on an expert each, all other picks
     outside the rank."""
     from conftest import pkg
     from test_plan import build_plan, wide_tile
 
     layer = pkg("moe_layer")
-    T, e_local = 3300, 16
+    T, e_local = 3456, 16
     inp = layer.build_moe_inputs(T=T, device="cuda", seed=T + len(routes))
     for k in ("gemm1_weights", "gemm1_weights_scale", "gemm2_weights", "gemm2_weights_scale"):
         inp[k] = inp[k][:e_local].contiguous()

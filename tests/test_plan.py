@@ -70,8 +70,8 @@ def test_stage2_decode_waves_on_256_cus(plan, T, e_local, waves):
 
 
 @pytest.mark.parametrize("T,e_local,wide", [
-    (3071, 32, 0), (3072, 32, 1), (3071, 17, 0), (3072, 17, 1), (3072, 16, 0), (3150, 16, 0), (3199, 16, 0),
-    (3200, 16, 1), (16384, 16, 1), (3200, 15, 0), (16384, 8, 0), (129, 32, 0)])
+    (3071, 32, 0), (3072, 32, 1), (3071, 17, 0), (3072, 17, 1), (3072, 16, 0), (3200, 16, 0), (3455, 16, 0),
+    (3456, 16, 1), (16384, 16, 1), (3456, 15, 0), (16384, 8, 0), (129, 32, 0)])
 def test_prefill_wide_on_256_cus(plan, T, e_local, wide):
     """The wide kernels' line: later where an item per weight block is at most
     one per CU."""
